@@ -121,7 +121,7 @@ struct Q8MulMat {
   const char* add = nullptr;
   int64_t add_nb0 = 0, add_nb1 = 0;
   // Optional activation prologue (streaming form only, q8_ring_form): instead
-  // of Q8_0_ACT blocks at `a`, each workgroup quantises the m F32 columns at x
+  // of Q8_0_ACT blocks at `a`, each workgroup quantises the F32 column at x
   // (x_ld floats apart) itself, after RMS_NORM * norm_w when norm_w is set
   // (src/ops_cpu.cpp:143-170) -- the separate norm / quantize launches fused.
   const float* x = nullptr;
@@ -152,7 +152,7 @@ __host__ __device__ inline int64_t q8_unperm_row(int64_t r, int32_t hd, int64_t 
   return head * hd + (w >> 1) + (w & 1) * (hd / 2);
 }
 // Whether launch_mul_mat_q8_0 takes the streaming form for p (the only form
-// with the activation prologue).
+// with the activation prologue, and that for one column only).
 bool q8_ring_form(const Q8MulMat& p);
 // Whether launch_mul_mat_q8_0 can run p with its SwiGLU epilogue (the
 // streaming form, one column, no added term or RoPE, n a multiple of 64 and
@@ -160,6 +160,8 @@ bool q8_ring_form(const Q8MulMat& p);
 bool q8_swiglu_out_ok(const Q8MulMat& p, int n_cu);
 hipError_t launch_quantize_q8_0_act(const Q8Quantize& p, hipStream_t stream);
 hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream);
+// mul_mat_cols.hip: several columns (Q8_0_ACT blocks at p.a, no prologue, RoPE or SwiGLU).
+hipError_t launch_mul_mat_q8_0_cols(const Q8MulMat& p, int n_cu, hipStream_t stream);
 
 // Cache append: src F32 [head_dim, n_head_kv, n_tokens] (device, byte strides)
 // into dst rows [pos0, pos0 + n_tokens) of a [head_dim, n_head_kv, n_ctx]

@@ -1,8 +1,9 @@
 // mul_mat.hip -- the step after attention on the device: MI_OP_QUANTIZE_Q8_0
 // (src/ops_cpu.cpp:462-479 -> src/quant.cpp:188-210) and MI_OP_MUL_MAT with
 // Q8_0 weights (src/ops_cpu.cpp:226-236), e.g. the attention output
-// projection. HBM-bound matrix-vector work: the weights are read once per
-// launch; a decode column reuses nothing else.
+// projection. This file has the quantiser and the products of one column
+// (HBM-bound: the weights are read once per launch and nothing is reused);
+// mul_mat_cols.hip has those of several.
 //
 // Both reproduce the engine bit for bit:
 //  - activation blocks of 32: amax by a strict greater-than scan, d = amax /
@@ -92,10 +93,7 @@ __global__ void quantize_q8_0_act_kernel(const Q8Quantize p) {
   }
 }
 
-// Rows of 8 lanes (32 rows per 256-thread workgroup); columns in chunks of
-// kQ8Cols, each lane keeping its accumulator for every column of the chunk.
-constexpr int kQ8Cols = 8;
-
+// One column, any alignment: rows of 8 lanes, 32 rows per 256-thread workgroup.
 __global__ __launch_bounds__(256) void mul_mat_q8_0_kernel(const Q8MulMat p) {
 #pragma clang fp contract(off)
   const int l = threadIdx.x & 7;
@@ -103,45 +101,30 @@ __global__ __launch_bounds__(256) void mul_mat_q8_0_kernel(const Q8MulMat p) {
   const bool live = row < p.n;  // dead lanes still join the exchanges
   const char* w = p.w + (live ? row : 0) * p.w_nb1;
   const int nblk = (int)(p.k / 32);
-  for (int64_t c0 = 0; c0 < p.m; c0 += kQ8Cols) {
-    const int nc = (int)min<int64_t>(kQ8Cols, p.m - c0);
-    float acc[kQ8Cols];
-#pragma unroll
-    for (int c = 0; c < kQ8Cols; ++c) acc[c] = 0.0f;
-    for (int b = 0; b < nblk; ++b) {
-      const char* wb = w + 34 * (int64_t)b;
-      // 34-byte blocks: the scale and the byte group are 2-byte aligned
-      const float wd = (float)__builtin_bit_cast(_Float16, gload<unsigned short>(wb));
-      const int wq = (int)((unsigned)gload<unsigned short>(wb + 2 + 4 * l) |
-                           ((unsigned)gload<unsigned short>(wb + 4 + 4 * l) << 16));
-#pragma unroll
-      for (int c = 0; c < kQ8Cols; ++c) {
-        if (c < nc) {
-          const char* ab = p.a + (c0 + c) * p.a_nb1 + 36 * (int64_t)b;
-          const float dxdy = wd * gload<float>(ab);
-          const int isum = __builtin_amdgcn_sdot4(wq, gload<int>(ab + 4 + 4 * l), 0, false);
-          acc[c] = __builtin_fmaf((float)isum, dxdy, acc[c]);
-        }
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < kQ8Cols; ++c) {
-      if (c < nc) {
-        // lanes l and l^4 -> acc_l + acc_(l+4); then pairs; lane 0 holds
-        // ((acc0 + acc4) + (acc1 + acc5)) + ((acc2 + acc6) + (acc3 + acc7))
-        float s = q8_hsum8(acc[c], threadIdx.x);
-        if (live && l == 0) {
-          if (p.add) s = s + gload<float>(p.add + row * p.add_nb0 + (c0 + c) * p.add_nb1);
-          gstore<float>(p.dst + q8_unperm_row(row, p.perm_hd, p.perm_rows) * p.dst_nb0 + (c0 + c) * p.dst_nb1, s);
-        }
-      }
-    }
+  float acc = 0.0f;
+  for (int b = 0; b < nblk; ++b) {
+    const char* wb = w + 34 * (int64_t)b;
+    // 34-byte blocks: the scale and the byte group are 2-byte aligned
+    const float wd = (float)__builtin_bit_cast(_Float16, gload<unsigned short>(wb));
+    const int wq = (int)((unsigned)gload<unsigned short>(wb + 2 + 4 * l) |
+                         ((unsigned)gload<unsigned short>(wb + 4 + 4 * l) << 16));
+    const char* ab = p.a + 36 * (int64_t)b;
+    const float dxdy = wd * gload<float>(ab);
+    const int isum = __builtin_amdgcn_sdot4(wq, gload<int>(ab + 4 + 4 * l), 0, false);
+    acc = __builtin_fmaf((float)isum, dxdy, acc);
+  }
+  // lanes l and l^4 -> acc_l + acc_(l+4); then pairs; lane 0 holds
+  // ((acc0 + acc4) + (acc1 + acc5)) + ((acc2 + acc6) + (acc3 + acc7))
+  float s = q8_hsum8(acc, threadIdx.x);
+  if (live && l == 0) {
+    if (p.add) s = s + gload<float>(p.add + row * p.add_nb0);
+    gstore<float>(p.dst + q8_unperm_row(row, p.perm_hd, p.perm_rows) * p.dst_nb0, s);
   }
 }
 
 // The streaming form, for weight rows of at most 1 KB (k <= 960: every matrix
-// of a 896-wide model), 16-byte aligned groups of 8 rows and M <= kQ8Cols
-// columns. One workgroup of 8 waves per CU; each wave walks row groups (8
+// of a 896-wide model), 16-byte aligned groups of 8 rows and one column (or
+// two of a very tall matrix: q8_ring_form). One workgroup of 8 waves per CU; each wave walks row groups (8
 // rows) g = wave_id, wave_id + stride, ... through a ring of 2 LDS slots
 // filled by buffer_load ... lds (16 bytes per lane, one resource per group
 // bounded at the tensor's end, so bytes past it arrive as zeros without a
@@ -153,10 +136,10 @@ constexpr int kQ8RowBytesMax = 1024;
 constexpr int kQ8RingWaves = 8;
 constexpr int kQ8Slot = 8 * kQ8RowBytesMax;
 constexpr int kQ8MaxBlocks = 30;                   // k <= 960
+constexpr int kQ8Cols = 2;
 constexpr int kQ8ActBytesMax = kQ8Cols * kQ8MaxBlocks * 36;
 constexpr int kQ8RingTake = kQ8RingWaves * 2 * kQ8Slot + kQ8ActBytesMax;  // the group counter
-constexpr int kQ8Scale = kQ8RingTake + 16;        // the norm scale of each column
-constexpr int kQ8RingLds = kQ8Scale + 4 * kQ8Cols;
+constexpr int kQ8RingLds = kQ8RingTake + 16;
 constexpr int kQ8XOff = kQ8RingLds;                // one F32 column's squares (M = 1), past the ring,
 constexpr int kQ8SqN = 8 * 128;                    // padded to the 8 waves' segments of 128
 constexpr int kQ8SumWork = kQ8XOff + 4 * kQ8SqN;   // the 8-wave ordered sum's work area
@@ -244,10 +227,6 @@ __global__ __launch_bounds__(kQ8RingWaves * kWave) void mul_mat_q8_0_ring_kernel
     return live ? g : -1;
   };
   int64_t g_0, g_1;  // the group in each slot, or -1
-  // LDS read through lds_t pointers into the regions past the ring: the
-  // compiler then sees that they cannot overlap the ring's LDS-direct
-  // requests and does not wait for those before reading
-  lds_t* const s_scale = lds + kQ8Scale;
   if constexpr (M == 1) {
     // One column: its loads go into registers (at most 2 elements, or 1
     // activation word, per thread: k <= 960), the ring's first requests
@@ -319,37 +298,9 @@ __global__ __launch_bounds__(kQ8RingWaves * kWave) void mul_mat_q8_0_ring_kernel
     if (p.swiglu_out && t < 32) lds_store<uint64_t>(lds + kQ8SwTab + 8 * t, te);
     wg_barrier();  // the activation (and expf's table) is staged
   } else {
-    if (!p.x) {
-      for (int i = threadIdx.x; i < M * abytes / 4; i += kQ8RingWaves * kWave) {
-        const int c = i / (abytes / 4), o = 4 * (i - c * (abytes / 4));
-        *reinterpret_cast<unsigned*>(act_lds + c * abytes + o) = gload<unsigned>(p.a + c * p.a_nb1 + o);
-      }
-    } else {
-      // the prologue: columns into LDS (the ring slots are free until the
-      // first refill), the norm's ordered sums, then one thread per element
-      // in groups of 32 lanes forming each block
-      float* const xs = reinterpret_cast<float*>(ring_lds);
-      float* const sq = xs + M * p.k;
-      const int k = (int)p.k;
-      for (int i = threadIdx.x; i < M * k; i += kQ8RingWaves * kWave) {
-        const int c = i / k;
-        const float v = gload<float>(p.x + c * p.x_ld + (i - c * k));
-        xs[i] = v;
-        sq[i] = v * v;
-      }
-      __syncthreads();
-      if (p.norm_w && threadIdx.x < M)
-        lds_store<float>(s_scale + 4 * threadIdx.x, rms_scale(ordered_sum(sq + threadIdx.x * k, k), k, p.eps));
-      __syncthreads();
-      for (int i = threadIdx.x; i < M * k; i += kQ8RingWaves * kWave) {
-        const int c = i / k, e = i - c * k;
-        const float y = p.norm_w ? (xs[i] * lds_load<float>(s_scale + 4 * c)) * gload<float>(p.norm_w + e) : xs[i];
-        float d;
-        const int q = q8_lane_quant(y, d);
-        char* blk = act_lds + c * abytes + 36 * (e / 32);
-        if ((e & 31) == 0) *reinterpret_cast<float*>(blk) = d;
-        blk[4 + (e & 31)] = (char)q;
-      }
+    for (int i = threadIdx.x; i < M * abytes / 4; i += kQ8RingWaves * kWave) {
+      const int c = i / (abytes / 4), o = 4 * (i - c * (abytes / 4));
+      *reinterpret_cast<unsigned*>(act_lds + c * abytes + o) = gload<unsigned>(p.a + c * p.a_nb1 + o);
     }
     if (threadIdx.x == 0) *take = 0u;
     __syncthreads();  // the activation is staged (before the ring requests: the barrier waits for all loads)
@@ -518,24 +469,19 @@ __global__ __launch_bounds__(kQ8RingWaves * kWave) void mul_mat_q8_0_ring_kernel
 }
 
 // The staged form, for rows longer than the ring's slots (e.g. a 4864-wide
-// FFN down projection) and for more than kQ8Cols columns (a prompt's
-// tokens): one wave per group of 8 rows copies the group's rows (contiguous
-// in memory) into LDS with 16-byte loads, then, per chunk of up to kQ8Cols
-// columns, stages the chunk's activation blocks beside them; lane (row r =
-// lane / 8, accumulator l = lane % 8) walks its row's blocks in order from
-// LDS. Weights are read from HBM once however many columns there are.
+// FFN down projection): one wave per group of 8 rows copies the group's rows
+// (contiguous in memory) and the column's activation blocks into LDS with
+// 16-byte loads; lane (row r = lane / 8, accumulator l = lane % 8) walks its
+// row's blocks in order from LDS.
 constexpr int kQ8StageLdsMax = 96 * 1024;
 
 __host__ __device__ inline int64_t round1k(int64_t n) { return (n + 1023) & ~int64_t(1023); }
-// LDS of the staged form: the 8-row group and one chunk of activation columns,
+// LDS of the staged form: the 8-row group and the activation column,
 // each rounded up to whole 1 KB LDS-direct transfers.
 __host__ __device__ inline int64_t q8_stage_lds_bytes(int64_t w_nb1, int64_t k) {
-  return round1k(8 * w_nb1) + round1k(kQ8Cols * (k / 32) * 36);
+  return round1k(8 * w_nb1) + round1k((k / 32) * 36);
 }
 
-// MC: columns per chunk (the host picks min(m, kQ8Cols)); only the last chunk
-// may be partial.
-template <int MC>
 __global__ __launch_bounds__(kWave) void mul_mat_q8_0_staged_kernel(const Q8MulMat p) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) char stage_lds[];
@@ -559,83 +505,54 @@ __global__ __launch_bounds__(kWave) void mul_mat_q8_0_staged_kernel(const Q8MulM
   const int nblk = (int)(p.k / 32);
   const int abytes = nblk * 36;
   const int64_t act_off = round1k(8 * p.w_nb1);
-  // contiguous 16-byte aligned columns: a chunk is one range, loaded the same way
-  const bool act_dma = p.a_nb1 == abytes && abytes % 16 == 0 && reinterpret_cast<uintptr_t>(p.a) % 16 == 0;
   const int l = lane & 7, r = lane >> 3;
   const int64_t row = g * 8 + r;
   const bool live = r < nrows;
   const lds_t* const w = lds + (live ? r : 0) * p.w_nb1;
-  for (int64_t c0 = 0; c0 < p.m; c0 += MC) {
-    const int nc = (int)min<int64_t>(MC, p.m - c0);
-    __syncthreads();  // the previous chunk's activation reads are done
-    if (act_dma) {
-      const int64_t bytes = (int64_t)nc * abytes;
-      const rsrc_t r = make_rsrc(p.a + c0 * p.a_nb1, (unsigned)bytes);
-      const int n1k = (int)((bytes + 1023) / 1024);
-      for (int i = 0; i < n1k; ++i)
-        dma16(r, (lds_t*)stage_lds + act_off + 1024 * i, (unsigned)(1024 * i + 16 * lane));
-    } else {
-      for (int i = lane; i < nc * abytes / 4; i += kWave) {
-        const int c = i / (abytes / 4), o = 4 * (i - c * (abytes / 4));
-        lds_store<unsigned>((lds_t*)(stage_lds + act_off + c * abytes + o),
-                            gload<unsigned>(p.a + (c0 + c) * p.a_nb1 + o));
-      }
-    }
-    // one column: the added term is requested now, so its latency overlaps
-    // the transfers'
-    float addv = 0.0f;
-    if (MC == 1 && p.add) addv = gload<float>(p.add + min(row, p.n - 1) * p.add_nb0 + c0 * p.add_nb1);
-    wait_vmem<0>();  // the LDS-direct transfers (and the added term) have landed
-    if (c0 == 0 && wb4 != wbytes && lane == 0)
-      lds_store<unsigned short>((lds_t*)(stage_lds + wb4), gload<unsigned short>(wsrc + wb4));
-    __syncthreads();
-    float acc[MC];
+  // a 16-byte aligned column of whole 16-byte groups: loaded the same way
+  if (abytes % 16 == 0 && reinterpret_cast<uintptr_t>(p.a) % 16 == 0) {
+    const rsrc_t ra = make_rsrc(p.a, (unsigned)abytes);
+    for (int i = 0; i < (abytes + 1023) / 1024; ++i)
+      dma16(ra, (lds_t*)stage_lds + act_off + 1024 * i, (unsigned)(1024 * i + 16 * lane));
+  } else {
+    for (int i = lane; i < abytes / 4; i += kWave)
+      lds_store<unsigned>((lds_t*)(stage_lds + act_off + 4 * i), gload<unsigned>(p.a + 4 * i));
+  }
+  // the added term is requested now, so its latency overlaps the transfers'
+  float addv = 0.0f;
+  if (p.add) addv = gload<float>(p.add + min(row, p.n - 1) * p.add_nb0);
+  wait_vmem<0>();  // the LDS-direct transfers (and the added term) have landed
+  if (wb4 != wbytes && lane == 0)
+    lds_store<unsigned short>((lds_t*)(stage_lds + wb4), gload<unsigned short>(wsrc + wb4));
+  __syncthreads();
+  float acc = 0.0f;
+  const lds_t* const act = lds + act_off;
+  // blocks in order; 8 at a time with all their LDS reads issued first, so
+  // their latency overlaps the chain of multiply-adds (a tail of fewer than
+  // 8 re-reads the last block and does not add it)
+  for (int b0 = 0; b0 < nblk; b0 += 8) {
+    float wd[8], ad[8];
+    int wq[8], aq[8];
 #pragma unroll
-    for (int c = 0; c < MC; ++c) acc[c] = 0.0f;
-    const lds_t* const act = lds + act_off + 4 + 4 * l;
-    // blocks in order; 8 at a time with all their LDS reads issued first, so
-    // their latency overlaps the chain of multiply-adds (a tail of fewer than
-    // 8 re-reads the last block and does not add it)
-    for (int b0 = 0; b0 < nblk; b0 += 8) {
-      float wd[8];
-      int wq[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const lds_t* wb = w + 34 * min(b0 + u, nblk - 1);
-        wd[u] = (float)__builtin_bit_cast(_Float16, lds_load<unsigned short>(wb));
-        wq[u] = (int)((unsigned)lds_load<unsigned short>(wb + 2 + 4 * l) |
-                      ((unsigned)lds_load<unsigned short>(wb + 4 + 4 * l) << 16));
-      }
-#pragma unroll
-      for (int c = 0; c < MC; ++c) {
-        if (MC == 1 || c < nc) {
-          float ad[8];
-          int aq[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            const int bb = min(b0 + u, nblk - 1);
-            ad[u] = lds_load<float>(act - 4 - 4 * l + c * abytes + 36 * bb);
-            aq[u] = lds_load<int>(act + c * abytes + 36 * bb);
-          }
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            const float r = __builtin_fmaf((float)__builtin_amdgcn_sdot4(wq[u], aq[u], 0, false),
-                                           wd[u] * ad[u], acc[c]);
-            acc[c] = b0 + u < nblk ? r : acc[c];
-          }
-        }
-      }
+    for (int u = 0; u < 8; ++u) {
+      const int bb = min(b0 + u, nblk - 1);
+      const lds_t* wb = w + 34 * bb;
+      wd[u] = (float)__builtin_bit_cast(_Float16, lds_load<unsigned short>(wb));
+      wq[u] = (int)((unsigned)lds_load<unsigned short>(wb + 2 + 4 * l) |
+                    ((unsigned)lds_load<unsigned short>(wb + 4 + 4 * l) << 16));
+      ad[u] = lds_load<float>(act + 36 * bb);
+      aq[u] = lds_load<int>(act + 36 * bb + 4 + 4 * l);
     }
 #pragma unroll
-    for (int c = 0; c < MC; ++c) {
-      if (MC == 1 || c < nc) {
-        float s = q8_hsum8(acc[c], threadIdx.x);
-        if (live && l == 0) {
-          if (p.add) s = s + (MC == 1 ? addv : gload<float>(p.add + row * p.add_nb0 + (c0 + c) * p.add_nb1));
-          gstore<float>(p.dst + q8_unperm_row(row, p.perm_hd, p.perm_rows) * p.dst_nb0 + (c0 + c) * p.dst_nb1, s);
-        }
-      }
+    for (int u = 0; u < 8; ++u) {
+      const float r = __builtin_fmaf((float)__builtin_amdgcn_sdot4(wq[u], aq[u], 0, false), wd[u] * ad[u], acc);
+      acc = b0 + u < nblk ? r : acc;
     }
+  }
+  float s = q8_hsum8(acc, threadIdx.x);
+  if (live && l == 0) {
+    if (p.add) s = s + addv;
+    gstore<float>(p.dst + q8_unperm_row(row, p.perm_hd, p.perm_rows) * p.dst_nb0, s);
   }
 }
 
@@ -751,12 +668,18 @@ bool q8_swiglu_out_ok(const Q8MulMat& p, int n_cu) {
          p.n / 64 <= (n_cu > 0 ? n_cu : 256) && q8_ring_form(p);
 }
 
+// Two columns only of a matrix tall enough that its bytes are what takes the
+// time (151936 x 896: 40.1 us against the column tiles' 47; 4864 x 896: 8.8
+// against 6.9; three columns of the tallest take 45 and 47).
+constexpr int64_t kQ8TwoColsRows = 65536;
+
 bool q8_ring_form(const Q8MulMat& p) {
   const bool act_ok = p.x ? (p.x_ld >= p.k && reinterpret_cast<uintptr_t>(p.x) % 4 == 0)
                           : (p.a_nb1 % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 4 == 0);
+  const bool cols_ok = p.m == 1 || (p.m == 2 && p.n >= kQ8TwoColsRows && !p.x && !p.perm_hd && !p.rope_on);
   // rows 4-byte aligned: every group's byte range ends on a whole dword (the
   // resource's range check is per dword)
-  return p.w_nb1 <= kQ8RowBytesMax && p.k <= 960 && p.m <= kQ8Cols && (8 * p.w_nb1) % 16 == 0 &&
+  return p.w_nb1 <= kQ8RowBytesMax && p.k <= 960 && cols_ok && (8 * p.w_nb1) % 16 == 0 &&
          p.w_nb1 % 4 == 0 &&
          reinterpret_cast<uintptr_t>(p.w) % 16 == 0 && act_ok && p.n * p.w_nb1 < (int64_t)1 << 40;
 }
@@ -766,20 +689,17 @@ hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) 
   const bool rows_form = q8_ring_form(p);
   if (p.x && !rows_form) return hipErrorInvalidValue;  // the prologue exists in the streaming form only
   if (rows_form) {
-    typedef void (*ring_fn)(const Q8MulMat);
-    static const ring_fn fns[2][kQ8Cols] = {
-        {mul_mat_q8_0_ring_kernel<1, false>, mul_mat_q8_0_ring_kernel<2, false>, mul_mat_q8_0_ring_kernel<3, false>,
-         mul_mat_q8_0_ring_kernel<4, false>, mul_mat_q8_0_ring_kernel<5, false>, mul_mat_q8_0_ring_kernel<6, false>,
-         mul_mat_q8_0_ring_kernel<7, false>, mul_mat_q8_0_ring_kernel<8, false>},
-        {mul_mat_q8_0_ring_kernel<1, true>, mul_mat_q8_0_ring_kernel<2, true>, mul_mat_q8_0_ring_kernel<3, true>,
-         mul_mat_q8_0_ring_kernel<4, true>, mul_mat_q8_0_ring_kernel<5, true>, mul_mat_q8_0_ring_kernel<6, true>,
-         mul_mat_q8_0_ring_kernel<7, true>, mul_mat_q8_0_ring_kernel<8, true>}};
+    const bool epi = p.rope_on || p.perm_hd;
+    const auto fn = p.m == 2 ? mul_mat_q8_0_ring_kernel<2, false>
+                    : epi    ? mul_mat_q8_0_ring_kernel<1, true>
+                             : mul_mat_q8_0_ring_kernel<1, false>;
     static const hipError_t attr = [] {
+      const void* fns[3] = {(const void*)&mul_mat_q8_0_ring_kernel<1, false>,
+                            (const void*)&mul_mat_q8_0_ring_kernel<1, true>,
+                            (const void*)&mul_mat_q8_0_ring_kernel<2, false>};
       hipError_t e = hipSuccess;
-      for (int v = 0; v < 2; ++v)
-        for (int m = 0; m < kQ8Cols; ++m)
-          if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)fns[v][m], hipFuncAttributeMaxDynamicSharedMemorySize, kQ8RingLdsAll);
+      for (const void* f : fns)
+        if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kQ8RingLdsAll);
       return e;
     }();
     if (attr != hipSuccess) return attr;
@@ -789,20 +709,12 @@ hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) 
     const unsigned grid = p.swiglu_out ? (unsigned)(p.n / 64)
                                        : (unsigned)std::min<int64_t>(n_cu > 0 ? n_cu : 256,
                                                                      (groups + kQ8RingWaves - 1) / kQ8RingWaves);
-    const bool epi = p.rope_on || p.perm_hd;
-    hipLaunchKernelGGL(fns[epi ? 1 : 0][p.m - 1], dim3(grid), dim3(kQ8RingWaves * kWave), kQ8RingLdsAll, stream, p);
-  } else if (q8_stage_lds_bytes(p.w_nb1, p.k) <= kQ8StageLdsMax &&
-             reinterpret_cast<uintptr_t>(p.w) % 16 == 0 && (8 * p.w_nb1) % 16 == 0 &&
-             p.a_nb1 % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 4 == 0) {
-    static const hipError_t attr = [] {
-      hipError_t e = hipSuccess;
-      const void* fns[2] = {(const void*)&mul_mat_q8_0_staged_kernel<1>,
-                            (const void*)&mul_mat_q8_0_staged_kernel<kQ8Cols>};
-      for (const void* f : fns)
-        if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kQ8StageLdsMax);
-      return e;
-    }();
-    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(kQ8RingWaves * kWave), kQ8RingLdsAll, stream, p);
+    return hipGetLastError();
+  }
+  if (p.m > 1) return launch_mul_mat_q8_0_cols(p, n_cu, stream);
+  if (q8_stage_lds_bytes(p.w_nb1, p.k) <= kQ8StageLdsMax && reinterpret_cast<uintptr_t>(p.w) % 16 == 0 &&
+      (8 * p.w_nb1) % 16 == 0 && p.a_nb1 % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 4 == 0) {
     const dim3 grid((unsigned)((p.n + 7) / 8));
     if (q8_s1_ok(p)) {
       static const hipError_t attr1 = hipFuncSetAttribute((const void*)&mul_mat_q8_0_staged1_kernel,
@@ -812,14 +724,13 @@ hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) 
                          (unsigned)q8_s1_lds_bytes(p.w_nb1, p.k), stream, p);
       return hipGetLastError();
     }
-    const unsigned lds = (unsigned)q8_stage_lds_bytes(p.w_nb1, p.k);
-    if (p.m == 1)
-      hipLaunchKernelGGL(mul_mat_q8_0_staged_kernel<1>, grid, dim3(kWave), lds, stream, p);
-    else
-      hipLaunchKernelGGL(mul_mat_q8_0_staged_kernel<kQ8Cols>, grid, dim3(kWave), lds, stream, p);
+    static const hipError_t attr = hipFuncSetAttribute((const void*)&mul_mat_q8_0_staged_kernel,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kQ8StageLdsMax);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL(mul_mat_q8_0_staged_kernel, grid, dim3(kWave), (unsigned)q8_stage_lds_bytes(p.w_nb1, p.k),
+                       stream, p);
   } else {
-    hipLaunchKernelGGL(mul_mat_q8_0_kernel, dim3((unsigned)((p.n + 31) / 32)), dim3(256), 0, stream,
-                       p);
+    hipLaunchKernelGGL(mul_mat_q8_0_kernel, dim3((unsigned)((p.n + 31) / 32)), dim3(256), 0, stream, p);
   }
   return hipGetLastError();
 }

@@ -123,3 +123,42 @@ def test_q8_0_strided_operands(hip, stream, oracle, k, n, m):
     assert np.array_equal(np.ascontiguousarray(a[:, :k // 32 * 36]).reshape(-1), want_act)
     want = oracle.mul_mat_q8_0(np.ascontiguousarray(w[:, :k // 32 * 34]), want_act, k, n, m)
     assert np.array_equal(bits(got), bits(want))
+
+
+@pytest.mark.parametrize("k,n,m", [
+    (32, 20, 5),       # one block per row
+    (96, 50, 33),      # fewer blocks than a stage, a column past a tile
+    (128, 1203, 131),  # one whole stage; tiles of 32 x 32, 19 rows and 3 columns left
+    (160, 4100, 16),   # a stage and a block; 16 columns, more rows than workgroups
+    (224, 900, 128),   # 7 blocks: the last stage re-reads one; tiles of 32 columns x 16 rows
+    (896, 33, 17),     # tiles of 16 x 16, one row and one column past
+    (4832, 47, 3),     # 151 blocks: the last stage re-reads one, of 38
+])
+def test_q8_0_columns_bitwise(hip, stream, oracle, k, n, m):
+    # Every tile shape of the several-column products, at its edges, against
+    # the oracle; and with activations so small that scale products and sums
+    # are denormal, against the one-column kernels (the oracle's host process
+    # may flush denormals).
+    import torch
+    rng = np.random.default_rng(k * 7 + n + m)
+    w = q8_weights(rng, n, k)
+    blocks = w.reshape(n, k // 32, 34)
+    blocks[0, :, :2] = (5, 0)        # fp16 denormal scales
+    blocks[-1, :, 2:10] = 0x80       # int8 -128, which no quantiser writes
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[m // 2] = 0.0
+    _, act, q = quantize_on_device(hip, stream, x)
+    got, _ = mul_mat_on_device(hip, stream, w, k, n, act, q, m)
+    want = oracle.mul_mat_q8_0(w, oracle.quantize_q8_0_act(x), k, n, m)
+    assert np.array_equal(bits(got), bits(want))
+
+    _, act, q = quantize_on_device(hip, stream, x * np.float32(1e-36))
+    got, dw = mul_mat_on_device(hip, stream, w, k, n, act, q, m)
+    one = torch.empty(n, device="cuda")
+    wt = make_tensor(dw.data_ptr(), [k, n], [34, w.shape[1]], type_=mh.MI_TYPE_Q8_0)
+    for j in {0, 1, m // 2, m - 1}:
+        qj = make_tensor(act.data_ptr() + j * (k // 32 * 36), [k, 1], [36, k // 32 * 36], type_=mh.MI_TYPE_Q8_0_ACT)
+        d = make_tensor(one.data_ptr(), [n, 1], [4, 4 * n], op=mh.MI_OP_MUL_MAT, src=[wt, qj])
+        hip.check(hip.mi_hip_op_mul_mat(ctypes.byref(d), stream))
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(got[j]), bits(one.cpu().numpy())), j
