@@ -9,18 +9,12 @@
 //   P_i  = e_i * (1 / sum)
 //   O[o] = sum_t V[o, kvh, t] * P_t            t ascending (masked t add +-0, skipped)
 //
-// Rows whose keys' V fit in LDS (a * head_dim * 4 <= kExactStageBytes) run
-// attn_exact_staged_kernel: 256 threads per (token j, head h); the row's K
-// rows come into LDS (LDS-direct, coalesced) and the threads form one key's
-// score each from there; then three waves bring the V rows over the K rows
-// while wave 0 forms the maximum, the exponentials and (lane 0) the ordered
-// sum; then each output element's lane runs its ordered V sum from LDS.
-// Longer rows run attn_exact_kernel: one wave
-// per (token, head), lanes splitting the keys and then the output elements,
-// V read from global memory. Either way the ordered sums make a row's cost
-// linear in its key count on one lane: this is the checking path for
-// whole-model parity (token ids equal to the reference engine's), not the
-// throughput path (decode.hip / prefill.hip).
+// The order leaves two chains of a dependent additions per row (8.4 cycles
+// each: 3.5 ns), the sum of the exponentials and an output element's sum;
+// everything else is independent and is taken off them. Few rows (a decode
+// step) run one workgroup per row, which shortens the chains
+// (attn_exact_row_kernel); many rows (a prompt) run several rows per wave,
+// which share the K and V tiles and fill the chip (attn_exact_tile_kernel).
 #include <cmath>
 
 #include "attn_common.h"
@@ -33,319 +27,562 @@ namespace mi {
 
 static __constant__ uint64_t kExpfTab[32] = MI_EXPF_TABLE;
 
-__global__ __launch_bounds__(kWave) void attn_exact_kernel(const ExactAttn p) {
+namespace {
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// 16 bytes per lane from each lane's address into LDS at lds + 16 * lane
+// (kept out of templates: the host pass drops a kernel template whose body
+// names the builtin directly).
+__device__ __forceinline__ void dma16_from(const char* p, lds_t* lds) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p,
+                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+// s + p[0] + p[1] + ... + p[n - 1] (n a multiple of 16, p 16-byte aligned), one
+// rounded addition each, in order; chunk c + 1 of 16 terms is read from LDS
+// between chunk c's additions (a dependent addition takes 8.4 cycles and
+// issues in 4.6, so the reads cost the chain nothing). Reads up to 16 floats
+// past n (never added).
+__device__ __forceinline__ float exact_sum(const lds_t* p, int n, float s) {
 #pragma clang fp contract(off)
-  extern __shared__ float prob[];
-  __shared__ float s_inv;
-  const int lane = threadIdx.x;
-  const int h = blockIdx.x % p.n_head;
-  const int j = blockIdx.x / p.n_head;
-  const int kvh = h / p.n_rep;
-  const int D = p.head_dim;
-  const int a = min(p.n_past + j + 1, p.n_past + p.n_tokens);
-  const float* q = reinterpret_cast<const float*>(p.q + h * p.q_s1 + (int64_t)j * p.q_s2);
-  float mx = -INFINITY;
-  for (int i = lane; i < a; i += kWave) {
-    const float* kr = reinterpret_cast<const float*>(p.k + kvh * p.k_s1 + (int64_t)i * p.k_s2);
-    float acc = 0.0f;
-#pragma unroll 16  // (the row's loads in flight together)
-    for (int d = 0; d < D; d += 4) {
-      const float4 kv = *reinterpret_cast<const float4*>(kr + d);
-      const float4 qv = *reinterpret_cast<const float4*>(q + d);
-      acc = acc + kv.x * qv.x;
-      acc = acc + kv.y * qv.y;
-      acc = acc + kv.z * qv.z;
-      acc = acc + kv.w * qv.w;
-    }
-    const float v = acc * p.scale;
-    prob[i] = v;
-    mx = v > mx ? v : mx;
-  }
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const float o = __shfl_xor(mx, off);
-    mx = o > mx ? o : mx;
-  }
-  for (int i = lane; i < a; i += kWave) prob[i] = expf_ref(prob[i] - mx, kExpfTab);
-  __syncthreads();
-  if (lane == 0) {
-    float sum = 0.0f;
-    for (int i = 0; i < a; ++i) sum = sum + prob[i];
-    s_inv = (float)(1.0 / (double)sum);  // the correctly rounded 1.0f / sum
-  }
-  __syncthreads();
-  const float inv = s_inv;
-  for (int i = lane; i < a; i += kWave) prob[i] = prob[i] * inv;
-  __syncthreads();
-  float* out = reinterpret_cast<float*>(p.out + h * p.o_s1 + (int64_t)j * p.o_s2);
-  const char* vbase = p.v + kvh * p.v_s1;
-  for (int o = lane; o < D; o += kWave) {
-    float acc = 0.0f;
-#pragma unroll 16  // (16 keys' loads in flight ahead of the ordered additions)
-    for (int t = 0; t < a; ++t)
-      acc = acc + *reinterpret_cast<const float*>(vbase + (int64_t)t * p.v_s2 + 4 * o) * prob[t];
-    out[o] = acc;
-  }
-}
-
-constexpr int kExactStageBytes = 128 * 1024;  // the staged kernel's V rows
-constexpr int kExactThreads = 256;
-
-// LDS of the staged kernel for rows of up to n_kv keys: the V rows (whole 1 KB
-// transfers), the probabilities, expf's table, the wave maxima and 1 / sum.
-// The V rows and the probabilities have 16 entries of room past n_kv: the
-// ordered sums read each chunk of 16 ahead of its additions, the one past
-// the last whole chunk too (read, never added).
-__host__ __device__ inline int exact_staged_vbytes(int n_kv, int d) {
-  return ((n_kv + 16) * d * 4 + 1023) & ~1023;
-}
-__host__ __device__ inline int exact_staged_lds(int n_kv, int d) {
-  return exact_staged_vbytes(n_kv, d) + 4 * (n_kv + 16) + 32 * 8 + 4 * 4 + 16;
-}
-
-// The ordered sums of the staged kernel, in chunks of 16 terms: chunk c + 1
-// is read from LDS before chunk c's additions, so that the chain of additions
-// does not wait for each read. Terms past the last whole chunk go one by one.
-// s + p[0] + p[1] + ... + p[n - 1] (p 16-byte aligned, 16 floats readable past n)
-__device__ __forceinline__ float exact_sum(const float* p, int n) {
-#pragma clang fp contract(off)
-  const float4* p4 = reinterpret_cast<const float4*>(p);
-  float s = 0.0f;
-  float4 x[4], y[4];
-  auto get = [&](float4 (&b)[4], int c) {
+  f32x4_t x[4], y[4];
+  auto get = [&](f32x4_t (&b)[4], int c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) b[u] = p4[4 * c + u];
+    for (int u = 0; u < 4; ++u) b[u] = lds_load<f32x4_t>(p + 64 * c + 16 * u);
   };
-  auto add = [&](const float4 (&b)[4]) {
+  auto add = [&](const f32x4_t (&b)[4], f32x4_t (&next)[4], int c) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       s = s + b[u].x;
+      next[u] = lds_load<f32x4_t>(p + 64 * c + 16 * u);
       s = s + b[u].y;
       s = s + b[u].z;
       s = s + b[u].w;
     }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);  // an addition
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
+      __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
   const int nch = n >> 4;
   get(x, 0);
   int c = 0;
-  // (the scheduler would otherwise sink each chunk's reads below the
-  // additions before them)
   for (; c + 1 < nch; c += 2) {
-    get(y, c + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    add(x);
-    get(x, c + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    add(y);
+    add(x, y, c + 1);
+    add(y, x, c + 2);
   }
-  if (c < nch) add(x);
-  for (int i = 16 * nch; i < n; ++i) s = s + p[i];
+  if (c < nch) add(x, y, c);
   return s;
 }
 
-// acc + v[0] * p[0] + v[D] * p[1] + ... + v[(n - 1) D] * p[n - 1], each
-// product and sum rounded (v: one output element's column of V rows D floats
-// apart; 16 rows and probabilities readable past n). The products do not
-// depend on the running sum: chunk c + 1's 16 are formed between chunk c's
-// additions, so each addition waits only for the one before it, not for a
-// multiplication issued just before it. (The same products, added in the
-// same order: the same bits.)
-template <int D>
-__device__ __forceinline__ float exact_dot(const float* v, const float* p, int n) {
+// acc + p[0] + p[S] + ... + p[(n - 1) S] (p in LDS, S floats apart), in order,
+// read two chunks of 16 ahead (a column of 64 lanes is 256 bytes a term: its
+// reads are further away than one chunk's additions). Reads rows up to the
+// next multiple of 16 past n (never added).
+template <int S>
+__device__ __forceinline__ float exact_column(const lds_t* p, int n, float acc) {
 #pragma clang fp contract(off)
-  const float4* p4 = reinterpret_cast<const float4*>(p);
-  float acc = 0.0f;
-  float va[16], vb[16];
-  float4 pa[4], pb[4];
-  float ra[16], rb[16];  // products
-  auto get = [&](float (&vv)[16], float4 (&pp)[4], int c) {
+  float x[3][16];
+  auto get = [&](float (&b)[16], int c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 16; ++u) vv[u] = v[(16 * c + u) * D];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) pp[u] = p4[4 * c + u];
+    for (int u = 0; u < 16; ++u) b[u] = lds_load<float>(p + 4 * S * (16 * c + u));
   };
-  auto prod = [&](float (&r)[16], const float (&vv)[16], const float4 (&pp)[4]) {
+  auto add = [&](const float (&b)[16], float (&next)[16], int c) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      r[4 * u] = vv[4 * u] * pp[u].x;
-      r[4 * u + 1] = vv[4 * u + 1] * pp[u].y;
-      r[4 * u + 2] = vv[4 * u + 2] * pp[u].z;
-      r[4 * u + 3] = vv[4 * u + 3] * pp[u].w;
+    for (int u = 0; u < 16; ++u) {
+      acc = acc + b[u];
+      next[u] = lds_load<float>(p + 4 * S * (16 * c + u));
     }
-  };
-  // chunk r's additions, chunk (vv, pp)'s products into rn between them
-  auto add_prod = [&](const float (&r)[16], float (&rn)[16], const float (&vv)[16], const float4 (&pp)[4]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      acc = acc + r[4 * u];
-      rn[4 * u] = vv[4 * u] * pp[u].x;
-      acc = acc + r[4 * u + 1];
-      rn[4 * u + 1] = vv[4 * u + 1] * pp[u].y;
-      acc = acc + r[4 * u + 2];
-      rn[4 * u + 2] = vv[4 * u + 2] * pp[u].z;
-      acc = acc + r[4 * u + 3];
-      rn[4 * u + 3] = vv[4 * u + 3] * pp[u].w;
+    for (int u = 0; u < 16; ++u) {
+      __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);  // an addition
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  auto add = [&](const float (&r)[16]) {
-#pragma unroll
-    for (int t = 0; t < 16; ++t) acc = acc + r[t];
-  };
-  const int nch = n >> 4;
-  if (nch > 0) {
-    get(va, pa, 0);
-    prod(ra, va, pa);
-    if (nch > 1) get(vb, pb, 1);
-    int c = 0;
-    // ra: chunk c's products; vb, pb: chunk c + 1's values
-    for (; c + 2 < nch; c += 2) {
-      get(va, pa, c + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      add_prod(ra, rb, vb, pb);
-      get(vb, pb, c + 3);  // (c + 3 <= nch: at most the chunk past the last whole one)
-      __builtin_amdgcn_sched_barrier(0);
-      add_prod(rb, ra, va, pa);
-    }
-    if (c + 1 < nch) {
-      add_prod(ra, rb, vb, pb);
-      add(rb);
-    } else {
-      add(ra);
-    }
+  const int nch = n >> 4, last = (n - 1) >> 4;  // whole chunks; the last chunk
+  get(x[0], 0);
+  get(x[1], min(1, last));
+  int c = 0;
+  for (; c + 2 < nch; c += 3) {
+    add(x[0], x[2], c + 2);
+    add(x[1], x[0], min(c + 3, last));
+    add(x[2], x[1], min(c + 4, last));
   }
-  for (int t = 16 * nch; t < n; ++t) acc = acc + v[t * D] * p[t];
+  if (c < nch) {
+    add(x[0], x[2], min(c + 2, last));
+    if (c + 1 < nch) add(x[1], x[0], min(c + 3, last));
+  }
+  for (int t = 16 * nch; t < n; ++t) acc = acc + lds_load<float>(p + 4 * S * t);
   return acc;
 }
 
-// D: head_dim (64 or 128). The row's K rows come into LDS first, into the
-// region that later holds its V rows: LDS-direct requests of whole 1 KB
-// (where a thread loading its own key row touches one cache line per lane
-// and instruction), 16-byte slots XOR-swizzled by row so that one row per
-// lane reads free of bank conflicts. After the scores, waves 1-3 bring the V
-// rows over the K rows while wave 0 forms the maximum, the exponentials and
-// the ordered sum; the barriers do not wait for vector memory (wg_barrier),
-// each wave waits for its own requests.
-template <int D>
-__global__ __launch_bounds__(kExactThreads) void attn_exact_staged_kernel(const ExactAttn p) {
+// Rows row0 .. row0 + n - 1 of one KV head (past `last`: row `last` again) into
+// LDS, n * D / 4 a multiple of 64, by NW waves of which this is the w-th: whole
+// 1 KB requests; 16-byte slots XOR-swizzled by row if SW, so that one row per
+// lane reads free of bank conflicts. A wave's requests are NW / 4 x 64 / D x 16
+// rows apart, where the swizzle repeats: an address is the one before plus a
+// constant.
+template <int D, int NW, bool SW>
+__device__ __forceinline__ void rows_to_lds(lds_t* dst, const char* base, int64_t s2, int row0, int n, int last,
+                                            int w, int lane) {
+  constexpr int PPR = D / 4;  // 16-byte pieces per row
+  constexpr int STEP = kWave * NW / PPR;
+  static_assert(!SW || STEP % 16 == 0, "the swizzle repeats every 16 rows");
+  const int r = (kWave * w + lane) / PPR, slot = lane % PPR;
+  const int col = 16 * (SW ? slot ^ swz<PPR>(r) : slot);
+  if (row0 + n - 1 <= last) {
+    const char* p = base + (int64_t)(row0 + r) * s2 + col;
+#pragma unroll
+    for (int i0 = kWave * w; i0 < n * PPR; i0 += kWave * NW) {
+      dma16_from(p, dst + 16 * i0);
+      p += STEP * s2;
+    }
+  } else {
+    for (int i0 = kWave * w, q = row0 + r; i0 < n * PPR; i0 += kWave * NW, q += STEP)
+      dma16_from(base + (int64_t)min(q, last) * s2 + col, dst + 16 * i0);
+  }
+}
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// One workgroup per (token, head).
+//
+// Scores: K rows come through two LDS buffers, one key per thread. The sum of
+// the exponentials is cut into 8 segments, one per wave, run from 64 candidate
+// start values each (as ordered_sum_lds_8waves states), so the chain is an
+// eighth as long. The output elements' chains are bare additions in one wave
+// (two at D = 128): four other waves form the products P_t V[t] into LDS, a
+// chunk ahead.
+//
+// Measured (14 / 2 heads, D 64, us per launch; before: one kernel with the
+// whole row in LDS up to 512 keys and one of a wave per row beyond): n_kv 129
+// 7.3 -> 6.7, 301 10.2 -> 8.0, 1501 75.8 -> 22.8. Of the 22.8 the output
+// chains take 10.5 (7 ns a key, 4.2 of them the addition itself), the scores
+// 6.7 (LDS-direct requests bring about 55 GB/s into a CU, and a row has one
+// CU), the exponentials and their sum 2.7.
+constexpr int kRowThreads = 512;
+constexpr int kRowWaves = kRowThreads / kWave;
+constexpr int kRowLoaders = 4;          // waves that form the products
+constexpr int kRowWork = 256 + 64 + 64 + kRowWaves * kWave * 4;  // expf's table, maxima, segment sums, ends
+constexpr int kLdsMax = 160 * 1024;
+
+// floats of the probabilities: 8 segments of whole 16s, 16 readable past them
+__host__ __device__ inline int row_segment(int n) { return ((n + 7) / 8 + 15) & ~15; }
+__host__ __device__ inline int row_prob_bytes(int n) { return 4 * (8 * row_segment(n) + 16); }
+inline int row_lds_bytes(int n, int buf) { return row_prob_bytes(n) + kRowWork + 2 * buf; }
+static_assert(4 * (kExactMaxKeys + 16) + kRowWork + 2 * 8 * 1024 <= kLdsMax, "the longest row fits");
+
+// BUF: bytes of a buffer of K rows (two, whole requests of every wave), later
+// of CK rows of products.
+template <int D, int BUF, int CK>
+__global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const ExactAttn p) {
 #pragma clang fp contract(off)
-  typedef float f32x4_t __attribute__((ext_vector_type(4)));
   extern __shared__ __attribute__((aligned(16))) char ex_lds[];
+  lds_t* const lds = (lds_t*)ex_lds;
+  constexpr int PPR = D / 4;
+  constexpr int KB = BUF / (4 * D);                       // keys per buffer
+  constexpr int kReq = BUF / (1024 * kRowWaves);          // requests per wave and buffer
+  static_assert(kReq * 1024 * kRowWaves == BUF && KB <= kRowThreads, "whole requests, a key per thread");
+  constexpr int NV = CK * PPR / (kRowLoaders * kWave);    // pieces of V per loader thread and buffer
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int h = blockIdx.x % p.n_head;
-  const int j = blockIdx.x / p.n_head;
+  const int j = p.n_tokens - 1 - blockIdx.x / p.n_head;  // the longest rows first
   const int kvh = h / p.n_rep;
-  const int a = min(p.n_past + j + 1, p.n_past + p.n_tokens);
-  const int n_kv = p.n_past + p.n_tokens;
-  const int vbytes = exact_staged_vbytes(n_kv, D);
-  constexpr int PPR = D / 4;  // 16-byte pieces per row
-  float* const vl = reinterpret_cast<float*>(ex_lds);  // K, later V, row t at vl + t D
-  float* const prob = reinterpret_cast<float*>(ex_lds + vbytes);
-  uint64_t* const tab = reinterpret_cast<uint64_t*>(ex_lds + vbytes + 4 * n_kv);
-  float* const red = reinterpret_cast<float*>(tab + 32);
-  const uint64_t te = kExpfTab[lane & 31];  // requested first: loads complete in order
-  const int pieces = a * PPR;
-  // rows of one KV head from base into LDS: piece i is physical slot i % PPR
-  // of row i / PPR, which holds logical slot (i % PPR) ^ sw(row); pieces past
-  // the row arrive as zeros. Waves w0.. w0 + nw - 1 share the requests.
-  auto rows_to_lds = [&](const char* base, int64_t s2, bool swizzle, int w0, int nw) __attribute__((always_inline)) {
-    const unsigned size = (unsigned)((int64_t)(a - 1) * s2 + 4 * D);
-    const rsrc_t r = make_rsrc(base, size);
-    for (int i0 = kWave * (wv - w0); i0 < pieces; i0 += kWave * nw) {
-      const int i = i0 + lane, row = i / PPR, slot = i % PPR;
-      const int ls = swizzle ? slot ^ swz<PPR>(row) : slot;
-      const unsigned off = i < pieces ? (unsigned)((int64_t)row * s2 + 16 * ls) : size;
-      dma16(r, (lds_t*)ex_lds + 16 * i0, off);
+  const int a = p.n_past + j + 1;
+  const int L = row_segment(a);
+  lds_t* const prob = lds;
+  lds_t* const tab = lds + row_prob_bytes(p.n_past + p.n_tokens);
+  lds_t* const red = tab + 256;
+  lds_t* const segsum = red + 64;
+  lds_t* const ends = segsum + 64;
+  lds_t* const buf = tab + kRowWork;
+  const char* const kbase = p.k + kvh * p.k_s1;
+  const char* const vbase = p.v + kvh * p.v_s1;
+  const uint64_t te = kExpfTab[lane & 31];
+  const float* q = reinterpret_cast<const float*>(p.q + h * p.q_s1 + (int64_t)j * p.q_s2);
+  f32x4_t qv[PPR];
+#pragma unroll
+  for (int u = 0; u < PPR; ++u) qv[u] = gload<f32x4_t>(q + 4 * u);
+  auto request = [&](int k0, int s, int n) __attribute__((always_inline)) {
+    rows_to_lds<D, kRowWaves, true>(buf + s * BUF, kbase, p.k_s2, k0, n, a - 1, wv, lane);
+  };
+  // one key's score, d ascending, product and sum each rounded
+  float mx = -INFINITY;
+  auto score = [&](int key, const lds_t* rowp, int row) __attribute__((always_inline)) {
+    float acc = 0.0f;
+    // 64 products first (they do not depend on one another), then their sum
+#pragma unroll
+    for (int u0 = 0; u0 < PPR; u0 += 16) {
+      f32x4_t pr[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const f32x4_t kv = lds_load<f32x4_t>(rowp + 16 * ((u0 + u) ^ swz<PPR>(row)));
+        pr[u] = f32x4_t{kv.x * qv[u0 + u].x, kv.y * qv[u0 + u].y, kv.z * qv[u0 + u].z, kv.w * qv[u0 + u].w};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        acc = acc + pr[u].x;
+        acc = acc + pr[u].y;
+        acc = acc + pr[u].z;
+        acc = acc + pr[u].w;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const float v = acc * p.scale;
+    lds_store<float>(prob + 4 * key, v);
+    mx = v > mx ? v : mx;
+  };
+  if (2 * KB <= kRowThreads && a <= 2 * KB) {
+    // both buffers at once, a key per thread (whole requests of 1 KB)
+    constexpr int kWhole = kWave / PPR;  // rows per request
+    const int n = (a + kWhole - 1) & ~(kWhole - 1);
+    request(0, 0, min(n, KB));
+    if (n > KB) request(KB, 1, n - KB);
+    wait_vmem<0>();
+    wg_barrier();
+    if (tid < a) score(tid, buf + tid * (4 * D), tid);  // (the buffers are adjacent)
+  } else {
+    request(0, 0, KB);
+    request(KB, 1, KB);  // (past the row: its last key, never used)
+    for (int k0 = 0, s = 0; k0 < a; k0 += KB, s ^= 1) {
+      wait_vmem<kReq>();  // this wave's requests for the buffer (and the query) have landed
+      wg_barrier();       // and everyone's
+      if (tid < KB && k0 + tid < a) score(k0 + tid, buf + s * BUF + tid * (4 * D), tid);
+      if (k0 + KB < a) {
+        wg_barrier();  // the buffer has been read
+        request(k0 + 2 * KB, s, KB);
+      }
+    }
+  }
+  if (tid < 32) lds_store<uint64_t>(tab + 8 * tid, te);
+  // the first V rows meanwhile, in the loaders' registers, two buffers ahead
+  // (waves 2, 3, 6 and 7: not on the SIMDs of the chains' waves 0 and 1)
+  const bool loader = (wv & 2) != 0;
+  const int lt = ((wv >> 2) * 2 + (wv & 1)) * kWave + lane;
+  f32x4_t vr[2][NV];
+  auto load_v = [&](f32x4_t (&x)[NV], int t0) __attribute__((always_inline)) {
+    constexpr int STEP = kRowLoaders * kWave / PPR;  // rows between a thread's pieces
+    const int r = t0 + lt / PPR;
+    if (t0 + CK <= a) {
+      const char* v = vbase + (int64_t)r * p.v_s2 + 16 * (lt % PPR);
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        x[u] = gload<f32x4_t>(v);
+        v += STEP * p.v_s2;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < NV; ++u)
+        x[u] = gload<f32x4_t>(vbase + (int64_t)min(r + u * STEP, a - 1) * p.v_s2 + 16 * (lt % PPR));
     }
   };
-  rows_to_lds(p.k + kvh * p.k_s1, p.k_s2, true, 0, kExactThreads / kWave);
-  // this wave's query elements into registers meanwhile
-  const float* q = reinterpret_cast<const float*>(p.q + h * p.q_s1 + (int64_t)j * p.q_s2);
-  float4 qv[PPR];
-#pragma unroll
-  for (int u = 0; u < PPR; ++u) qv[u] = *reinterpret_cast<const float4*>(q + 4 * u);
-  wait_vmem<0>();  // this wave's K requests (and the query) have landed
-  wg_barrier();
-  // one key's score per thread, d ascending, product and sum each rounded
-  float mx = -INFINITY;
-  for (int i = tid; i < a; i += kExactThreads) {
-    const lds_t* const rowp = (const lds_t*)ex_lds + i * (4 * D);
-    // the D products first (independent), then their sum in order
-    float pr[D];
-#pragma unroll
-    for (int u = 0; u < PPR; ++u) {
-      const f32x4_t kv = lds_load<f32x4_t>(rowp + 16 * (u ^ swz<PPR>(i)));
-      pr[4 * u] = kv.x * qv[u].x;
-      pr[4 * u + 1] = kv.y * qv[u].y;
-      pr[4 * u + 2] = kv.z * qv[u].z;
-      pr[4 * u + 3] = kv.w * qv[u].w;
-    }
-    float acc = 0.0f;
-#pragma unroll
-    for (int d = 0; d < D; ++d) acc = acc + pr[d];
-    const float v = acc * p.scale;
-    prob[i] = v;
-    mx = v > mx ? v : mx;
+  if (loader) {
+    load_v(vr[0], 0);
+    load_v(vr[1], CK);
   }
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    const float o = __shfl_xor(mx, off);
+  mx = wave_max_dpp(mx);  // (never NaN; the sign of a zero maximum changes no exponential)
+  if (lane == 0) lds_store<float>(red + 4 * wv, mx);
+  wg_barrier();  // the scores and the waves' maxima
+  mx = lds_load<float>(red);
+#pragma unroll
+  for (int w = 1; w < kRowWaves; ++w) {
+    const float o = lds_load<float>(red + 4 * w);
     mx = o > mx ? o : mx;
   }
-  if (tid < 32) tab[tid] = te;
-  if (lane == 0) red[wv] = mx;
-  wg_barrier();  // the scores are in LDS and every K row has been read
-  if (wv > 0) {
-    rows_to_lds(p.v + kvh * p.v_s1, p.v_s2, false, 1, kExactThreads / kWave - 1);
-    wait_vmem<0>();  // this wave's V requests have landed
-  } else {
-    mx = red[0];
-    for (int w = 1; w < kExactThreads / kWave; ++w) mx = red[w] > mx ? red[w] : mx;
-    for (int i = lane; i < a; i += kWave) prob[i] = expf_ref(prob[i] - mx, tab);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's exponentials are in LDS
-    if (lane == 0) {
-      const float sum = exact_sum(prob, a);
-      red[4] = (float)(1.0 / (double)sum);  // the correctly rounded 1.0f / sum
+  // each wave its segment's exponentials, and their sum in double, which
+  // places the candidates
+  lds_t* const seg = prob + 4 * L * wv;
+  double qs = 0.0;
+  for (int i = lane; i < L; i += kWave) {
+    const float x = lds_load<float>(seg + 4 * i) - mx;
+    const float e = L * wv + i < a ? expf_ref(x, (const __attribute__((address_space(3))) uint64_t*)tab) : 0.0f;
+    lds_store<float>(seg + 4 * i, e);
+    qs += (double)e;
+  }
+  qs = wave_sum_f64(qs);
+  if (lane == 0) lds_store<double>(segsum + 8 * wv, qs);
+  wg_barrier();
+  int base[kRowWaves];
+  double pre = 0.0;
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) {
+    const int gb = __builtin_bit_cast(int, (float)pre);
+    base[w] = gb > 32 ? gb - 32 : 0;
+    pre += lds_load<double>(segsum + 8 * w);
+  }
+  int my_base = base[0];
+#pragma unroll
+  for (int w = 1; w < kRowWaves; ++w) my_base = wv == w ? base[w] : my_base;
+  lds_store<float>(ends + 4 * (kWave * wv + lane), exact_sum(seg, L, __builtin_bit_cast(float, my_base + lane)));
+  wg_barrier();
+  float e[kRowWaves], sum = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) e[w] = lds_load<float>(ends + 4 * (kWave * w + lane));
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) {
+    const int c = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, sum) - base[w]);
+    if (c >= 0 && c < kWave)
+      sum = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e[w]), c));
+    else
+      sum = exact_sum(prob + 4 * L * w, L, sum);
+  }
+  const float inv = (float)(1.0 / (double)sum);  // the correctly rounded 1.0f / sum
+  // products by the loaders, chains by the first waves, a buffer apart
+  if (tid < D) __builtin_amdgcn_s_setprio(3);
+  float acc = 0.0f;
+  auto chunk = [&](int t0, f32x4_t (&x)[NV], lds_t* b) __attribute__((always_inline)) {
+    if (loader) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const int i = u * kRowLoaders * kWave + lt, row = i / PPR;
+        const float pt = lds_load<float>(prob + 4 * min(t0 + row, a - 1)) * inv;
+        lds_store<f32x4_t>(b + 16 * i, f32x4_t{x[u].x * pt, x[u].y * pt, x[u].z * pt, x[u].w * pt});
+      }
+      load_v(x, t0 + 2 * CK);
+    }
+    wg_barrier();
+    if (tid < D) acc = exact_column<D>(b + 4 * tid, min(CK, a - t0), acc);
+  };
+  for (int t0 = 0; t0 < a; t0 += 2 * CK) {
+    chunk(t0, vr[0], buf);
+    if (t0 + CK < a) chunk(t0 + CK, vr[1], buf + BUF);
+  }
+  if (tid < D) reinterpret_cast<float*>(p.out + h * p.o_s1 + (int64_t)j * p.o_s2)[tid] = acc;
+}
+
+// ---------------------------------------------------------------------------
+// Many rows: the T n_rep rows (token, head) of one KV head, R consecutive ones
+// per wave, W waves per workgroup. Tiles of 64 keys come through two LDS
+// buffers, first all of K, then all of V, each request a tile ahead. Per tile
+// a wave forms its rows' scores with one key per lane (the queries are
+// uniform: scalar loads), later its rows' sums with one output element per
+// lane (two at D = 128); in between, lane r runs row r's ordered sum.
+//
+// The vector units and LDS reads bound it: two vector instructions per product
+// (the order forbids the fused one), 4 D per (row, key) in all, and every
+// operand of them read from LDS or through scalar loads. Measured (14 / 2
+// heads, D 64, us; before: a workgroup with its own copy of K and V per row):
+// 128 tokens 11.2 -> 7.9, 384 tokens 123.8 -> 20.1.
+constexpr int kTileKeys = 64;
+// floats per row of scores: whole tiles, plus 4 so that the rows of a wave
+// start in different banks (and 16 readable past the last)
+__host__ __device__ inline int tile_row_floats(int n) { return ((n + 63) & ~63) + 4; }
+template <int D, int W, int R>
+constexpr int tile_lds_bytes(int n) {
+  return 2 * kTileKeys * D * 4 + 256 + 4 * W * R * tile_row_floats(n) + 64;
+}
+
+template <int D, int W, int R>
+__global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAttn p, int n_tiles) {
+#pragma clang fp contract(off)
+  extern __shared__ __attribute__((aligned(16))) char ex_lds[];
+  lds_t* const lds = (lds_t*)ex_lds;
+  constexpr int PPR = D / 4, kBuf = kTileKeys * D * 4, ND = D / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int n_hkv = p.n_head / p.n_rep;
+  const int kvh = blockIdx.x % n_hkv;
+  const int n_rows = p.n_tokens * p.n_rep;
+  const int tile = n_tiles - 1 - blockIdx.x / n_hkv;  // the longest rows first
+  const int np = tile_row_floats(p.n_past + p.n_tokens);
+  lds_t* const tab = lds + 2 * kBuf;
+  lds_t* const sc = tab + 256 + 4 * np * R * wv;  // this wave's rows
+  const char* const kbase = p.k + kvh * p.k_s1;
+  const char* const vbase = p.v + kvh * p.v_s1;
+  // the wave's rows (past the last: the last again, not stored) and their keys
+  const int r0 = (tile * W + wv) * R;
+  int a[R];
+  const char* q[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = min(r0 + i, n_rows - 1), j = r / p.n_rep, h = kvh * p.n_rep + (r - j * p.n_rep);
+    a[i] = p.n_past + j + 1;
+    q[i] = p.q + h * p.q_s1 + (int64_t)j * p.q_s2;
+  }
+  const int a_lo = a[0], a_hi = a[R - 1];  // a wave's rows have ascending key counts
+  const int a_wg = p.n_past + min((tile + 1) * W * R - 1, n_rows - 1) / p.n_rep + 1;
+  const int nt = (a_wg + kTileKeys - 1) / kTileKeys;
+  const uint64_t te = kExpfTab[lane & 31];
+  if (tid < 32) lds_store<uint64_t>(tab + 8 * tid, te);
+  auto request = [&](int s) __attribute__((always_inline)) {
+    lds_t* const b = lds + (s & 1) * kBuf;
+    if (s < nt)
+      rows_to_lds<D, W, true>(b, kbase, p.k_s2, s * kTileKeys, kTileKeys, a_wg - 1, wv, lane);
+    else
+      rows_to_lds<D, W, false>(b, vbase, p.v_s2, (s - nt) * kTileKeys, kTileKeys, a_wg - 1, wv, lane);
+  };
+  request(0);
+  float mx[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) mx[i] = -INFINITY;
+  for (int s = 0; s < nt; ++s) {
+    wait_vmem<0>();
+    wg_barrier();  // tile s has landed, and everyone has left the other buffer
+    request(s + 1);
+    const int k0 = s * kTileKeys;
+    if (k0 >= a_hi) continue;
+    const lds_t* const rowp = lds + (s & 1) * kBuf + lane * (4 * D);
+    float acc[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc[i] = 0.0f;
+#pragma unroll
+    for (int u0 = 0; u0 < PPR; u0 += 4) {
+      f32x4_t kv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) kv[u] = lds_load<f32x4_t>(rowp + 16 * ((u0 + u) ^ swz<PPR>(lane)));
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          // uniform address: a scalar load
+          const f32x4_t qv = *(const __attribute__((address_space(4))) f32x4_t*)(q[i] + 16 * (u0 + u));
+          acc[i] = acc[i] + kv[u].x * qv.x;
+          acc[i] = acc[i] + kv[u].y * qv.y;
+          acc[i] = acc[i] + kv[u].z * qv.z;
+          acc[i] = acc[i] + kv[u].w * qv.w;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const float v = acc[i] * p.scale;
+      lds_store<float>(sc + 4 * (i * np + k0 + lane), v);
+      mx[i] = k0 + lane < a[i] && v > mx[i] ? v : mx[i];
     }
   }
-  wg_barrier();  // the V rows and 1 / sum
-  const float inv = red[4];
-  for (int i = tid; i < a; i += kExactThreads) prob[i] = prob[i] * inv;
-  wg_barrier();
-  if (tid < D) {
-    const float acc = exact_dot<D>(vl + tid, prob, a);
-    float* out = reinterpret_cast<float*>(p.out + h * p.o_s1 + (int64_t)j * p.o_s2);
-    out[tid] = acc;
+  // exponentials, zeros past a row's keys (they leave its sum unchanged)
+  const int n_pad = (a_hi + 15) & ~15;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    mx[i] = wave_max_dpp(mx[i]);  // (never NaN; the sign of a zero maximum changes no exponential)
+    for (int t = lane; t < n_pad; t += kWave) {
+      const float x = lds_load<float>(sc + 4 * (i * np + t)) - mx[i];
+      lds_store<float>(sc + 4 * (i * np + t),
+                       t < a[i] ? expf_ref(x, (const __attribute__((address_space(3))) uint64_t*)tab) : 0.0f);
+    }
+  }
+  wave_lds_fence();
+  const float sum = exact_sum(sc + 4 * np * min(lane, R - 1), n_pad, 0.0f);
+  const float inv_l = (float)(1.0 / (double)sum);  // the correctly rounded 1.0f / sum
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const float inv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv_l), i));
+    for (int t = lane; t < n_pad; t += kWave)
+      lds_store<float>(sc + 4 * (i * np + t), lds_load<float>(sc + 4 * (i * np + t)) * inv);
+  }
+  wave_lds_fence();
+  float acc[R][ND];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int d = 0; d < ND; ++d) acc[i][d] = 0.0f;
+  for (int s = 0; s < nt; ++s) {
+    wait_vmem<0>();
+    wg_barrier();
+    if (s + 1 < nt) request(nt + s + 1);
+    const int k0 = s * kTileKeys;
+    const lds_t* const vb = lds + ((nt + s) & 1) * kBuf + 4 * lane;
+    const lds_t* const pb = sc + 4 * k0;
+    // keys every row of the wave sees, 4 at a time, then the others one by one
+    const int n4 = max(min(a_lo - k0, kTileKeys), 0) >> 2, n1 = min(a_hi - k0, kTileKeys);
+#pragma unroll 4
+    for (int t4 = 0; t4 < n4; ++t4) {
+      float v[4][ND];
+      f32x4_t pr[R];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int d = 0; d < ND; ++d) v[t][d] = lds_load<float>(vb + (4 * t4 + t) * (4 * D) + 4 * kWave * d);
+#pragma unroll
+      for (int i = 0; i < R; ++i) pr[i] = lds_load<f32x4_t>(pb + 4 * (i * np + 4 * t4));
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int d = 0; d < ND; ++d) acc[i][d] = acc[i][d] + v[t][d] * pr[i][t];
+    }
+    for (int t = 4 * n4; t < n1; ++t) {
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        if (k0 + t < a[i]) {
+          const float pt = lds_load<float>(pb + 4 * (i * np + t));
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            acc[i][d] = acc[i][d] + lds_load<float>(vb + t * (4 * D) + 4 * kWave * d) * pt;
+        }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = r0 + i;
+    if (r < n_rows) {
+      const int j = r / p.n_rep, h = kvh * p.n_rep + (r - j * p.n_rep);
+      float* const out = reinterpret_cast<float*>(p.out + h * p.o_s1 + (int64_t)j * p.o_s2);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) gstore<float>(out + kWave * d + lane, acc[i][d]);
+    }
   }
 }
 
-hipError_t launch_attn_exact(const ExactAttn& p, hipStream_t stream) {
-  const int n_kv = p.n_past + p.n_tokens;
-  if ((int64_t)n_kv * p.head_dim * 4 <= kExactStageBytes && (p.head_dim == 64 || p.head_dim == 128) &&
-      p.v_s2 % 4 == 0 && reinterpret_cast<uintptr_t>(p.v) % 4 == 0 && p.v_s1 % 4 == 0) {
-    static const hipError_t attr = [] {
-      hipError_t e = hipFuncSetAttribute((const void*)&attn_exact_staged_kernel<64>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         exact_staged_lds(kExactStageBytes / (4 * 64), 64));
-      if (e == hipSuccess)
-        e = hipFuncSetAttribute((const void*)&attn_exact_staged_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                exact_staged_lds(kExactStageBytes / (4 * 128), 128));
-      return e;
-    }();
-    if (attr != hipSuccess) return attr;
-    const dim3 grid((unsigned)(p.n_tokens * p.n_head));
-    const size_t lds = (size_t)exact_staged_lds(n_kv, p.head_dim);
-    if (p.head_dim == 64)
-      hipLaunchKernelGGL(attn_exact_staged_kernel<64>, grid, dim3(kExactThreads), lds, stream, p);
-    else
-      hipLaunchKernelGGL(attn_exact_staged_kernel<128>, grid, dim3(kExactThreads), lds, stream, p);
-    return hipGetLastError();
-  }
-  const size_t lds = (size_t)n_kv * sizeof(float);
-  static const hipError_t attr = hipFuncSetAttribute(
-      (const void*)&attn_exact_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kExactMaxKeys * 4);
+template <int D, int BUF, int CK>
+static hipError_t launch_row(const ExactAttn& p, hipStream_t stream) {
+  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_row_kernel<D, BUF, CK>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(attn_exact_kernel, dim3((unsigned)(p.n_tokens * p.n_head)), dim3(kWave), lds,
-                     stream, p);
+  hipLaunchKernelGGL((attn_exact_row_kernel<D, BUF, CK>), dim3((unsigned)(p.n_tokens * p.n_head)), dim3(kRowThreads),
+                     (unsigned)row_lds_bytes(p.n_past + p.n_tokens, BUF), stream, p);
   return hipGetLastError();
+}
+template <int D>
+static hipError_t launch_row(const ExactAttn& p, hipStream_t stream) {
+  // the largest buffers that fit beside the probabilities; short rows start
+  // their chains after half as many products
+  const int n_kv = p.n_past + p.n_tokens;
+  if (n_kv <= 512) return launch_row<D, 64 * 1024, 4096 / D>(p, stream);
+  if (row_lds_bytes(n_kv, 64 * 1024) <= kLdsMax) return launch_row<D, 64 * 1024, 8192 / D>(p, stream);
+  if (row_lds_bytes(n_kv, 32 * 1024) <= kLdsMax) return launch_row<D, 32 * 1024, 8192 / D>(p, stream);
+  return launch_row<D, 8 * 1024, 2048 / D>(p, stream);
+}
+
+template <int D, int W, int R>
+static hipError_t launch_tile(const ExactAttn& p, hipStream_t stream) {
+  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_tile_kernel<D, W, R>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
+  if (attr != hipSuccess) return attr;
+  const int rows = p.n_tokens * p.n_rep;
+  const int n_tiles = (rows + W * R - 1) / (W * R);
+  const unsigned lds = (unsigned)tile_lds_bytes<D, W, R>(p.n_past + p.n_tokens);
+  hipLaunchKernelGGL((attn_exact_tile_kernel<D, W, R>), dim3((unsigned)(n_tiles * (p.n_head / p.n_rep))),
+                     dim3(W * kWave), lds, stream, p, n_tiles);
+  return hipGetLastError();
+}
+
+// One row per wave: 128 tokens of 14 heads 7.9 us with 8 waves of 1 row, 10.1
+// with 8 of 2, 8.3 with 4 of 1; 384 tokens 20.1, 23.8 and 19.5.
+constexpr int kTileWaves = 8, kTileRows = 1;
+
+template <int D>
+static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
+  const int n_kv = p.n_past + p.n_tokens;
+  const int64_t rows = (int64_t)p.n_tokens * p.n_head;
+  // Rows that get a CU each take a workgroup each (14 rows of 1501 keys: 22.8
+  // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.9 us, 41 a row
+  // per workgroup), unless their scores do not fit in LDS (about 4000 keys).
+  if (rows <= n_cu || tile_lds_bytes<D, kTileWaves, kTileRows>(n_kv) > kLdsMax) return launch_row<D>(p, stream);
+  return launch_tile<D, kTileWaves, kTileRows>(p, stream);
+}
+
+hipError_t launch_attn_exact(const ExactAttn& p, int n_cu, hipStream_t stream) {
+  n_cu = n_cu > 0 ? n_cu : 256;
+  return p.head_dim == 64 ? launch<64>(p, n_cu, stream) : launch<128>(p, n_cu, stream);
 }
 
 }  // namespace mi

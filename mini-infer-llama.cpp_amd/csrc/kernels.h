@@ -171,7 +171,7 @@ hipError_t launch_kv_append(char* dst, int64_t dst_s1, int64_t dst_s2, bool dst_
                             int n_head_kv, int pos0, int n_tokens, hipStream_t stream);
 
 // attn_exact.hip: the attention triple in the reference's operation order
-// (F32 K/V, head_dim a multiple of 4, n_past + n_tokens <= kExactMaxKeys).
+// (F32 K/V, head_dim 64 or 128, n_past + n_tokens <= kExactMaxKeys).
 constexpr int kExactMaxKeys = 32768;
 struct ExactAttn {
   const char* q;  // [head_dim, n_head, n_tokens], byte strides q_s1 (head), q_s2 (token)
@@ -182,7 +182,7 @@ struct ExactAttn {
   int32_t n_head, n_rep, n_past, n_tokens, head_dim;
   float scale;
 };
-hipError_t launch_attn_exact(const ExactAttn& p, hipStream_t stream);
+hipError_t launch_attn_exact(const ExactAttn& p, int n_cu, hipStream_t stream);
 
 // Host helpers of the library's entry points (runtime.hip), for the other
 // host files: the thread's last-error message, the accounted device

@@ -676,7 +676,7 @@ int enqueue_forward(mi_hip_qwen2* m, const int32_t* ids_dev, int T, int n_past, 
       ea.n_tokens = T;
       ea.head_dim = hd;
       ea.scale = scale;
-      Q2_TRY(mi::launch_attn_exact(ea, st), "reference-order attention launch");
+      Q2_TRY(mi::launch_attn_exact(ea, mi::rt_n_cu(), st), "reference-order attention launch");
     } else if ((rc = mi_hip_attn_fwd(&aa))) {
       return rc;
     }

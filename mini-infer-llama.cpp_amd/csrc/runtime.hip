@@ -1299,7 +1299,7 @@ int mi_hip_attn_fwd_reference_order(const mi_hip_attn_args* a) {
   ea.n_tokens = a->n_tokens;
   ea.head_dim = r.head_dim;
   ea.scale = a->scale;
-  const hipError_t e = mi::launch_attn_exact(ea, static_cast<hipStream_t>(a->stream));
+  const hipError_t e = mi::launch_attn_exact(ea, g.n_cu, static_cast<hipStream_t>(a->stream));
   return e == hipSuccess ? MI_HIP_OK : hip_fail(e, "reference-order attention launch");
 }
 

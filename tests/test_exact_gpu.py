@@ -118,3 +118,18 @@ def test_random_shapes_bit_for_bit(hip, stream, case):
     q, k, v = _inputs(3000 + i, n_tok, n_past + n_tok, hkv * n_rep, hkv, d)
     _check(hip, stream, q, k, v, n_past, scale,
            f"random case {i}: n_head_kv {hkv} n_rep {n_rep} D {d} n_past {n_past} n_tokens {n_tok}")
+
+
+@pytest.mark.parametrize("hkv,n_rep,d,n_past,n_tok", [
+    (2, 7, 64, 8200, 1),     # one row per workgroup: half-size K buffers (past 7,000 keys)
+    (1, 2, 64, 24500, 1),    # and the smallest ones
+    (2, 2, 128, 513, 2),     # a buffer more than both hold at head_dim 128
+    (1, 1, 64, 0, 300),      # more rows than workgroups: tiles, from one key up
+    (2, 7, 64, 63, 37),      # key counts across a tile's edge, rows past the last
+    (3, 5, 128, 60, 20),     # head_dim 128, 100 rows per KV head
+    (1, 8, 64, 4300, 40),    # more rows than workgroups, scores too long for tiles
+])
+def test_row_and_tile_kernels_bit_for_bit(hip, stream, hkv, n_rep, d, n_past, n_tok):
+    q, k, v = _inputs(77 + n_past, n_tok, n_past + n_tok, hkv * n_rep, hkv, d)
+    _check(hip, stream, q, k, v, n_past, float(np.float32(d ** -0.5)),
+           f"{hkv} x {n_rep} heads of {d}, {n_tok} rows after {n_past}")
