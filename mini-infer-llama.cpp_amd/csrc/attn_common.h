@@ -238,6 +238,22 @@ __device__ inline float wave_max_dpp(float x) {
 // order; this stops the compiler from moving them across the point).
 __device__ inline void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
+// Reads one dword of each 128-byte line of [p, p + bytes), n threads together
+// (this is thread t), so that the lines are in the XCD's L2 for a later reader.
+__device__ __forceinline__ void warm_lines(const char* p, int64_t bytes, int t, int n) {
+  constexpr int kFlight = 8;
+  for (int64_t o = 128 * (int64_t)t; o < bytes; o += 128 * (int64_t)n * kFlight) {
+    unsigned x[kFlight];
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) {
+      const int64_t q = o + 128 * (int64_t)n * u;
+      x[u] = gload<unsigned>(p + (q < bytes ? q : o));
+    }
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) asm volatile("" ::"v"(x[u]));
+  }
+}
+
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 
 // Four consecutive cache elements as float4 (F32: one 16-byte load; F16: one

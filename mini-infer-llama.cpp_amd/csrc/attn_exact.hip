@@ -15,6 +15,7 @@
 // step) run one workgroup per row, which shortens the chains
 // (attn_exact_row_kernel); many rows (a prompt) run several rows per wave,
 // which share the K and V tiles and fill the chip (attn_exact_tile_kernel).
+#include <algorithm>
 #include <cmath>
 
 #include "attn_common.h"
@@ -138,7 +139,6 @@ __device__ __forceinline__ void rows_to_lds(lds_t* dst, const char* base, int64_
   const int col = 16 * (SW ? slot ^ swz<PPR>(r) : slot);
   if (row0 + n - 1 <= last) {
     const char* p = base + (int64_t)(row0 + r) * s2 + col;
-#pragma unroll
     for (int i0 = kWave * w; i0 < n * PPR; i0 += kWave * NW) {
       dma16_from(p, dst + 16 * i0);
       p += STEP * s2;
@@ -192,6 +192,22 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
   constexpr int NV = CK * PPR / (kRowLoaders * kWave);    // pieces of V per loader thread and buffer
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // every parameter in one round of scalar loads, not one where each is first used
+  asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.q_s1), "s"(p.q_s2), "s"(p.k_s1), "s"(p.k_s2), "s"(p.v_s1),
+               "s"(p.v_s2), "s"(p.n_head), "s"(p.n_rep), "s"(p.n_past), "s"(p.n_tokens), "s"(p.scale));
+  const int n_rows = p.n_tokens * p.n_head;
+  if ((int)blockIdx.x >= n_rows) {
+    // a workgroup past the rows: its share of what the next launches read,
+    // pieces of its own XCD (the same workgroup number modulo 8)
+    const int xcd = blockIdx.x % 8, first = (n_rows + 7 - xcd) / 8, per_xcd = ((int)gridDim.x + 7 - xcd) / 8 - first;
+    for (int w = 0, c = blockIdx.x / 8 - first; w < kMaxWarmUps; ++w) {
+      const int n = (p.warm[w].n + 7 - xcd) / 8;  // pieces of this XCD
+      for (; c < n; c += per_xcd)
+        warm_lines(p.warm[w].p + (int64_t)(xcd + 8 * c) * p.warm[w].bytes, p.warm[w].bytes, tid, kRowThreads);
+      c -= n;
+    }
+    return;
+  }
   const int h = blockIdx.x % p.n_head;
   const int j = p.n_tokens - 1 - blockIdx.x / p.n_head;  // the longest rows first
   const int kvh = h / p.n_rep;
@@ -246,9 +262,20 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
     const int n = (a + kWhole - 1) & ~(kWhole - 1);
     request(0, 0, min(n, KB));
     if (n > KB) request(KB, 1, n - KB);
-    wait_vmem<0>();
+    // V is asked for only after the scores: a dword of each of its 128-byte
+    // lines now, so that they are in L2 by then
+    constexpr int kLines = D / 32, kTouch = (2 * KB * kLines + kRowThreads - 1) / kRowThreads;
+    unsigned vt[kTouch];
+#pragma unroll
+    for (int u = 0; u < kTouch; ++u) {
+      const int i = min(tid + u * kRowThreads, a * kLines - 1);
+      vt[u] = gload<unsigned>(vbase + (int64_t)(i / kLines) * p.v_s2 + 128 * (i % kLines));
+    }
+    wait_vmem<kTouch>();  // the K rows
     wg_barrier();
     if (tid < a) score(tid, buf + tid * (4 * D), tid);  // (the buffers are adjacent)
+#pragma unroll
+    for (int u = 0; u < kTouch; ++u) asm volatile("" ::"v"(vt[u]));
   } else {
     request(0, 0, KB);
     request(KB, 1, KB);  // (past the row: its last key, never used)
@@ -533,23 +560,28 @@ __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAt
 }
 
 template <int D, int BUF, int CK>
-static hipError_t launch_row(const ExactAttn& p, hipStream_t stream) {
+static hipError_t launch_row(const ExactAttn& p, int n_cu, hipStream_t stream) {
   static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_row_kernel<D, BUF, CK>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((attn_exact_row_kernel<D, BUF, CK>), dim3((unsigned)(p.n_tokens * p.n_head)), dim3(kRowThreads),
+  // what is to be warmed up gets the idle CUs, two pieces each
+  const int rows = p.n_tokens * p.n_head;
+  int64_t pieces = 0;
+  for (const WarmUp& w : p.warm) pieces += w.n;
+  const int side = (int)std::min<int64_t>(std::max(n_cu - rows, 0) & ~7, (pieces + 15) / 16 * 8);
+  hipLaunchKernelGGL((attn_exact_row_kernel<D, BUF, CK>), dim3((unsigned)(rows + side)), dim3(kRowThreads),
                      (unsigned)row_lds_bytes(p.n_past + p.n_tokens, BUF), stream, p);
   return hipGetLastError();
 }
 template <int D>
-static hipError_t launch_row(const ExactAttn& p, hipStream_t stream) {
+static hipError_t launch_row(const ExactAttn& p, int n_cu, hipStream_t stream) {
   // the largest buffers that fit beside the probabilities; short rows start
   // their chains after half as many products
   const int n_kv = p.n_past + p.n_tokens;
-  if (n_kv <= 512) return launch_row<D, 64 * 1024, 4096 / D>(p, stream);
-  if (row_lds_bytes(n_kv, 64 * 1024) <= kLdsMax) return launch_row<D, 64 * 1024, 8192 / D>(p, stream);
-  if (row_lds_bytes(n_kv, 32 * 1024) <= kLdsMax) return launch_row<D, 32 * 1024, 8192 / D>(p, stream);
-  return launch_row<D, 8 * 1024, 2048 / D>(p, stream);
+  if (n_kv <= 512) return launch_row<D, 64 * 1024, 4096 / D>(p, n_cu, stream);
+  if (row_lds_bytes(n_kv, 64 * 1024) <= kLdsMax) return launch_row<D, 64 * 1024, 8192 / D>(p, n_cu, stream);
+  if (row_lds_bytes(n_kv, 32 * 1024) <= kLdsMax) return launch_row<D, 32 * 1024, 8192 / D>(p, n_cu, stream);
+  return launch_row<D, 8 * 1024, 2048 / D>(p, n_cu, stream);
 }
 
 template <int D, int W, int R>
@@ -576,7 +608,7 @@ static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
   // Rows that get a CU each take a workgroup each (14 rows of 1501 keys: 22.8
   // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.9 us, 41 a row
   // per workgroup), unless their scores do not fit in LDS (about 4000 keys).
-  if (rows <= n_cu || tile_lds_bytes<D, kTileWaves, kTileRows>(n_kv) > kLdsMax) return launch_row<D>(p, stream);
+  if (rows <= n_cu || tile_lds_bytes<D, kTileWaves, kTileRows>(n_kv) > kLdsMax) return launch_row<D>(p, n_cu, stream);
   return launch_tile<D, kTileWaves, kTileRows>(p, stream);
 }
 

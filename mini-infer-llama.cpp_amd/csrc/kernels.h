@@ -142,6 +142,13 @@ struct Q8MulMat {
   // With rope_on (streaming form, m = 1): the RopeEpi stores replace dst's.
   int32_t rope_on = 0;
   RopeEpi rope{};
+  // With rope_on, optional: two ranges of warm_bytes that the launch after this
+  // one reads on every XCD (the layer's cached K and V rows), brought into the
+  // L2s by workgroups on idle CUs.
+  const char* warm[2] = {nullptr, nullptr};
+  int64_t warm_bytes = 0;
+  // Set by the launcher: workgroups of the matrix itself (streaming form).
+  int32_t n_wg = 0;
 };
 
 // The natural row of stored row r of a matrix whose first perm_rows rows are
@@ -173,6 +180,15 @@ hipError_t launch_kv_append(char* dst, int64_t dst_s1, int64_t dst_s2, bool dst_
 // attn_exact.hip: the attention triple in the reference's operation order
 // (F32 K/V, head_dim 64 or 128, n_past + n_tokens <= kExactMaxKeys).
 constexpr int kExactMaxKeys = 32768;
+// Memory that the launches after this one read: `n` pieces of `bytes` from p,
+// piece b by workgroup b of its launch. Workgroups are dealt to the 8 XCDs in
+// turn, so a workgroup with the same number modulo 8 here can bring the piece
+// into the L2 that will be asked for it.
+struct WarmUp {
+  const char* p;
+  int32_t bytes, n;
+};
+constexpr int kMaxWarmUps = 4;
 struct ExactAttn {
   const char* q;  // [head_dim, n_head, n_tokens], byte strides q_s1 (head), q_s2 (token)
   const char* k;  // cache rows: k_s1 (KV head), k_s2 (position)
@@ -181,6 +197,9 @@ struct ExactAttn {
   int64_t q_s1, q_s2, k_s1, k_s2, v_s1, v_s2, o_s1, o_s2;
   int32_t n_head, n_rep, n_past, n_tokens, head_dim;
   float scale;
+  // Optional (one-workgroup-per-row launches only): brought into L2 by the CUs
+  // that the rows leave idle.
+  WarmUp warm[kMaxWarmUps] = {};
 };
 hipError_t launch_attn_exact(const ExactAttn& p, int n_cu, hipStream_t stream);
 

@@ -190,6 +190,22 @@ __global__ __launch_bounds__(kQ8RingWaves * kWave) void mul_mat_q8_0_ring_kernel
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) char ring_lds[];
   lds_t* const lds = (lds_t*)ring_lds;
+  // every parameter of the prologue in one round of scalar loads, not one
+  // round where each is first used
+  if constexpr (M == 1)
+    asm volatile("" ::"s"(p.w), "s"(p.a), "s"(p.w_nb1), "s"(p.k), "s"(p.n), "s"(p.x), "s"(p.norm_w), "s"(p.eps),
+                 "s"(p.swiglu_out), "s"(p.add), "s"(p.dst), "s"(p.n_wg));
+  if constexpr (EPI) {
+    if ((int)blockIdx.x >= p.n_wg) {
+      // a workgroup past the matrix: its share, among those of its XCD (the
+      // same number modulo 8), of the ranges to be warmed up
+      const int xcd = blockIdx.x % 8, first = (p.n_wg + 7 - xcd) / 8;
+      const int of = ((int)gridDim.x + 7 - xcd) / 8 - first, t = (blockIdx.x / 8 - first) * blockDim.x + threadIdx.x;
+      warm_lines(p.warm[0], p.warm_bytes, t, of * blockDim.x);
+      warm_lines(p.warm[1], p.warm_bytes, t, of * blockDim.x);
+      return;
+    }
+  }
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int nblk = (int)(p.k / 32);
@@ -199,8 +215,8 @@ __global__ __launch_bounds__(kQ8RingWaves * kWave) void mul_mat_q8_0_ring_kernel
   // from an LDS counter as they refill, so a wave served faster takes more
   // and the waves finish together.
   const int64_t n_groups = (p.n + 7) / 8;
-  const int64_t glo = n_groups * blockIdx.x / gridDim.x;
-  const int64_t ngw = n_groups * (blockIdx.x + 1) / gridDim.x - glo;
+  const int64_t glo = n_groups * blockIdx.x / p.n_wg;
+  const int64_t ngw = n_groups * (blockIdx.x + 1) / p.n_wg - glo;
   __attribute__((address_space(3))) unsigned* const take =
       reinterpret_cast<__attribute__((address_space(3))) unsigned*>(lds + kQ8RingTake);
   const int64_t total = p.n * p.w_nb1;
@@ -578,6 +594,9 @@ __global__ __launch_bounds__(kQ8S1Waves * kWave) void mul_mat_q8_0_staged1_kerne
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) char stage_lds[];
   const lds_t* const lds = (const lds_t*)stage_lds;
+  // (the parameters in one round of scalar loads)
+  asm volatile("" ::"s"(p.w), "s"(p.a), "s"(p.w_nb1), "s"(p.k), "s"(p.n), "s"(p.add), "s"(p.add_nb0), "s"(p.dst),
+               "s"(p.dst_nb0), "s"(p.perm_hd));
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int64_t g = blockIdx.x;
@@ -709,7 +728,14 @@ hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) 
     const unsigned grid = p.swiglu_out ? (unsigned)(p.n / 64)
                                        : (unsigned)std::min<int64_t>(n_cu > 0 ? n_cu : 256,
                                                                      (groups + kQ8RingWaves - 1) / kQ8RingWaves);
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(kQ8RingWaves * kWave), kQ8RingLdsAll, stream, p);
+    Q8MulMat q = p;
+    q.n_wg = (int32_t)grid;
+    // 64 KB per workgroup and XCD
+    const unsigned side = epi && p.warm_bytes > 0
+                              ? 8 * (unsigned)std::min<int64_t>((p.warm_bytes * 2 + 65535) / 65536,
+                                                                std::max((n_cu > 0 ? n_cu : 256) - (int)grid, 0) / 8)
+                              : 0;
+    hipLaunchKernelGGL(fn, dim3(grid + side), dim3(kQ8RingWaves * kWave), kQ8RingLdsAll, stream, q);
     return hipGetLastError();
   }
   if (p.m > 1) return launch_mul_mat_q8_0_cols(p, n_cu, stream);

@@ -536,6 +536,12 @@ int proj(const mi_hip_qwen2* m, const char* w, int64_t row_bytes, int64_t n, int
     if (p.x && m_cols == 1 && mi::q8_ring_form(p)) {
       p.rope_on = 1;
       p.rope = *rope;
+      // the cached rows [0, pos) of this layer's K and V, position-major: a
+      // step reads more weights than the caches hold, so attention would find
+      // them in HBM (24 layers, 300 keys: 1003 -> 965 us a token)
+      p.warm_bytes = (int64_t)rope->pos * m->kvd * 4;
+      p.warm[0] = rope->k_row - p.warm_bytes;
+      p.warm[1] = rope->v_row - p.warm_bytes;
     } else {
       p.perm_hd = rope->hd;
       p.perm_rows = (int64_t)rope->n_q + rope->n_kv;
@@ -567,6 +573,12 @@ int quantize_cols(const mi_hip_qwen2* m, const float* src, int64_t ne0, int64_t 
   p.rows = cols;
   hipError_t e = mi::launch_quantize_q8_0_act(p, m->stream);
   return e == hipSuccess ? MI_HIP_OK : mi::rt_hip_fail(e, "qwen2 quantize launch");
+}
+
+// The rows of a matrix as the one-column streaming form deals them to its
+// workgroups (64 each while there are fewer of those than CUs).
+mi::WarmUp q8_warm_up(const char* w, int64_t row_bytes, int64_t rows) {
+  return {w, (int32_t)(64 * row_bytes), rows / 64 <= mi::rt_n_cu() ? (int32_t)(rows / 64) : 0};
 }
 
 // Enqueues one forward pass on the model's stream, nothing waited for: the T
@@ -676,6 +688,14 @@ int enqueue_forward(mi_hip_qwen2* m, const int32_t* ids_dev, int T, int n_past, 
       ea.n_tokens = T;
       ea.head_dim = hd;
       ea.scale = scale;
+      if (T == 1) {
+        // the CUs without a head bring the next matrices into L2 (together
+        // with one round of parameter loads per launch 1048 -> 1003 us a token)
+        ea.warm[0] = q8_warm_up(w.wo, m->row_e, E);
+        ea.warm[1] = q8_warm_up(w.wgu, m->row_e, 2 * (int64_t)F);
+        ea.warm[2] = {w.wdown, (int32_t)(8 * m->row_f), E / 8};
+        if (l + 1 < hp.n_layer) ea.warm[3] = q8_warm_up(m->layers[l + 1].wqkv, m->row_e, qkv_rows);
+      }
       Q2_TRY(mi::launch_attn_exact(ea, mi::rt_n_cu(), st), "reference-order attention launch");
     } else if ((rc = mi_hip_attn_fwd(&aa))) {
       return rc;
