@@ -123,6 +123,20 @@ __device__ __forceinline__ float exact_column(const lds_t* p, int n, float acc) 
   return acc;
 }
 
+// Output element o (its lane's, in aligned groups of 32 lanes) of row (j, h).
+__device__ __forceinline__ void store_out(const ExactAttn& p, int j, int h, int o, float v) {
+  if (p.aq) {
+    float d;
+    const int q = q8_lane_quant(v, d);
+    const int e = h * p.head_dim + o;
+    char* const blk = p.aq + (int64_t)j * p.aq_ld + 36 * (e / 32);
+    if ((e & 31) == 0) gstore<float>(blk, d);
+    gstore<signed char>(blk + 4 + (e & 31), (signed char)q);
+  } else {
+    gstore<float>(p.out + h * p.o_s1 + (int64_t)j * p.o_s2 + 4 * o, v);
+  }
+}
+
 // Rows row0 .. row0 + n - 1 of one KV head (past `last`: row `last` again) into
 // LDS, n * D / 4 a multiple of 64, by NW waves of which this is the w-th: whole
 // 1 KB requests; 16-byte slots XOR-swizzled by row if SW, so that one row per
@@ -382,7 +396,7 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
     chunk(t0, vr[0], buf);
     if (t0 + CK < a) chunk(t0 + CK, vr[1], buf + BUF);
   }
-  if (tid < D) reinterpret_cast<float*>(p.out + h * p.o_s1 + (int64_t)j * p.o_s2)[tid] = acc;
+  if (tid < D) store_out(p, j, h, tid, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -552,9 +566,8 @@ __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAt
     const int r = r0 + i;
     if (r < n_rows) {
       const int j = r / p.n_rep, h = kvh * p.n_rep + (r - j * p.n_rep);
-      float* const out = reinterpret_cast<float*>(p.out + h * p.o_s1 + (int64_t)j * p.o_s2);
 #pragma unroll
-      for (int d = 0; d < ND; ++d) gstore<float>(out + kWave * d + lane, acc[i][d]);
+      for (int d = 0; d < ND; ++d) store_out(p, j, h, kWave * d + lane, acc[i][d]);
     }
   }
 }

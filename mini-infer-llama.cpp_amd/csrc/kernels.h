@@ -94,18 +94,20 @@ struct Q8Quantize {
   int64_t src_nb[4], dst_nb[4];
   int64_t ne0, ne1, ne2, rows;  // rows = ne1 * ne2 * ne3
 };
-// RoPE and the K/V append as the epilogue of the stacked Q/K/V projection
-// (one column): rows are n_q Q rows then n_kv K rows then n_kv V rows, Q and K
+// RoPE and the K/V append as the epilogue of the stacked Q/K/V projection:
+// rows are n_q Q rows then n_kv K rows then n_kv V rows, Q and K
 // rows permuted within each head of hd rows so that row 2j holds dim j and row
 // 2j + 1 dim j + hd/2 (a rotation pair in one 8-row group). Q lands roped in
 // natural order at q_out, K roped and V as is in the cache rows of position
 // pos (element (head h, dim d) at k_row / v_row + h * c_s1 + 4 d).
+// With several columns, column j is position pos + j: its Q at q_out + j *
+// q_ld, its K and V at k_row / v_row + j * c_s2.
 struct RopeEpi {
   const float* cs;  // (cos, sin) pairs, float2 at [pos * hd/2 + j]
   float* q_out;
   char* k_row;
   char* v_row;
-  int64_t c_s1;
+  int64_t c_s1, c_s2, q_ld;
   int32_t pos, hd, n_q, n_kv;
 };
 
@@ -139,7 +141,8 @@ struct Q8MulMat {
   // RopeEpi describes; the stores put them back in natural order (0: none).
   int32_t perm_hd = 0;
   int64_t perm_rows = 0;
-  // With rope_on (streaming form, m = 1): the RopeEpi stores replace dst's.
+  // With rope_on (streaming form with m = 1, or several columns): the RopeEpi
+  // stores replace dst's.
   int32_t rope_on = 0;
   RopeEpi rope{};
   // With rope_on, optional: two ranges of warm_bytes that the launch after this
@@ -167,7 +170,7 @@ bool q8_ring_form(const Q8MulMat& p);
 bool q8_swiglu_out_ok(const Q8MulMat& p, int n_cu);
 hipError_t launch_quantize_q8_0_act(const Q8Quantize& p, hipStream_t stream);
 hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream);
-// mul_mat_cols.hip: several columns (Q8_0_ACT blocks at p.a, no prologue, RoPE or SwiGLU).
+// mul_mat_cols.hip: several columns (Q8_0_ACT blocks at p.a, no prologue or SwiGLU).
 hipError_t launch_mul_mat_q8_0_cols(const Q8MulMat& p, int n_cu, hipStream_t stream);
 
 // Cache append: src F32 [head_dim, n_head_kv, n_tokens] (device, byte strides)
@@ -197,6 +200,11 @@ struct ExactAttn {
   int64_t q_s1, q_s2, k_s1, k_s2, v_s1, v_s2, o_s1, o_s2;
   int32_t n_head, n_rep, n_past, n_tokens, head_dim;
   float scale;
+  // Optional: the output as Q8_0_ACT blocks (element h * head_dim + o of token j
+  // in block (h * head_dim + o) / 32 of the column at aq + j * aq_ld) instead of
+  // F32 at out -- the engine's QUANTIZE node before the output projection fused.
+  char* aq = nullptr;
+  int64_t aq_ld = 0;
   // Optional (one-workgroup-per-row launches only): brought into L2 by the CUs
   // that the rows leave idle.
   WarmUp warm[kMaxWarmUps] = {};

@@ -31,6 +31,7 @@
 namespace mi {
 namespace {
 
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
@@ -106,18 +107,51 @@ __device__ __forceinline__ void stage_fma(float (&acc)[4 * NQ][4], const f16x4_t
   for (int l = 0; l < 4 * NQ; ++l) asm volatile("" : "+v"(acc[l][0]), "+v"(acc[l][1]), "+v"(acc[l][2]), "+v"(acc[l][3]));
 }
 
-// (row, 4 columns from col): one lane's finished outputs
+// (row, 4 columns from col): one lane's finished outputs. Lane c has row `row`,
+// lane c ^ 1 the other row of its RoPE pair (stored rows 2j and 2j + 1).
 __device__ __forceinline__ void store_cols(const Q8MulMat& p, int64_t row, int64_t col, const float (&out)[4]) {
-  if (row >= p.n) return;
-  char* const d = p.dst + q8_unperm_row(row, p.perm_hd, p.perm_rows) * p.dst_nb0;
+#pragma clang fp contract(off)
+  const bool live = row < p.n;
+  float v[4];
   const char* const ad = p.add + row * p.add_nb0;
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    if (col + r < p.m) {
-      float v = out[r];
-      if (p.add) v = v + gload<float>(ad + (col + r) * p.add_nb1);
-      gstore<float>(d + (col + r) * p.dst_nb1, v);
+  for (int r = 0; r < 4; ++r) v[r] = p.add && live && col + r < p.m ? out[r] + gload<float>(ad + (col + r) * p.add_nb1) : out[r];
+  char* d;
+  int64_t step;
+  if (p.rope_on) {
+    const RopeEpi& re = p.rope;
+    const int r0 = (int)row, qk_rows = re.n_q + re.n_kv, h = r0 / re.hd, w = r0 - h * re.hd;
+    float other[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) other[r] = dpp_mov<0xB1>(v[r]);  // quad_perm [1,0,3,2]
+    if (!live) return;
+    const bool odd = w & 1;
+    if (r0 < qk_rows) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (col + r < p.m) {
+          const f32x2_t cs = gload<f32x2_t>(re.cs + 2 * ((re.pos + col + r) * (re.hd / 2) + w / 2));
+          const float c = cs.x, s = cs.y;
+          const float x0 = odd ? other[r] : v[r], x1 = odd ? v[r] : other[r];
+          v[r] = odd ? x0 * s + x1 * c : x0 * c - x1 * s;
+        }
     }
+    const int e = r0 < qk_rows ? (w >> 1) + odd * (re.hd / 2) : w;
+    if (r0 < re.n_q) {
+      d = reinterpret_cast<char*>(re.q_out + h * re.hd + e);
+      step = 4 * re.q_ld;
+    } else {
+      d = (r0 < qk_rows ? re.k_row + (h - re.n_q / re.hd) * re.c_s1 : re.v_row + (h - qk_rows / re.hd) * re.c_s1) + 4 * e;
+      step = re.c_s2;
+    }
+  } else {
+    if (!live) return;
+    d = p.dst + q8_unperm_row(row, p.perm_hd, p.perm_rows) * p.dst_nb0;
+    step = p.dst_nb1;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (col + r < p.m) gstore<float>(d + (col + r) * step, v[r]);
 }
 
 }  // namespace
@@ -373,6 +407,10 @@ static hipError_t launch_tile(Q8MulMat p, hipStream_t stream) {
     if (e != hipSuccess) return e;
     p.a += step * p.a_nb1;
     p.dst += step * p.dst_nb1;
+    p.rope.pos += (int32_t)step;
+    p.rope.q_out += step * p.rope.q_ld;
+    p.rope.k_row += step * p.rope.c_s2;
+    p.rope.v_row += step * p.rope.c_s2;
     if (p.add) p.add += step * p.add_nb1;
   }
   return hipSuccess;

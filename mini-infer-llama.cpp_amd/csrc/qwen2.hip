@@ -96,6 +96,44 @@ __global__ __launch_bounds__(kNormThreads) void norm_q8_kernel(const float* x, i
   }
 }
 
+// The same for columns of at most 1024 elements: the ordered sum by 8 waves
+// together (ordered_sum_lds_8waves, the same bits), two elements per thread
+// kept in registers. 128 columns of 896: 8.0 -> 4.5 us (a launch that does next
+// to nothing takes about 4 here).
+constexpr int kNormWideMaxE = 1024;
+__global__ __launch_bounds__(512) void norm_q8_8waves_kernel(const float* x, int64_t x_ld, const float* w, float eps,
+                                                             char* aq, int64_t aq_ld, int E) {
+#pragma clang fp contract(off)
+  __shared__ __attribute__((aligned(16))) char sq[4 * kNormWideMaxE];
+  __shared__ __attribute__((aligned(16))) char work[64 + 8 * kWave * 4];
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(t / kWave);
+  const float* xr = x + (int64_t)blockIdx.x * x_ld;
+  float v[2] = {0.0f, 0.0f}, nw[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (t + 512 * j < E) {
+      v[j] = gload<float>(xr + t + 512 * j);
+      nw[j] = gload<float>(w + t + 512 * j);
+    }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) lds_store<float>((lds_t*)sq + 4 * (t + 512 * j), v[j] * v[j]);
+  wg_barrier();
+  const float scale =
+      rms_scale(ordered_sum_lds_8waves<kNormWideMaxE / 8>((const lds_t*)sq, (lds_t*)work, wv, lane), E, eps);
+  char* dst = aq + (int64_t)blockIdx.x * aq_ld;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int i = t + 512 * j;
+    if (i < E) {  // E % 32 == 0: whole 32-lane groups
+      float d;
+      const int q = q8_lane_quant((v[j] * scale) * nw[j], d);
+      if ((i & 31) == 0) gstore<float>(dst + 36 * (i / 32), d);
+      gstore<signed char>(dst + 36 * (i / 32) + 4 + (i & 31), (signed char)q);
+    }
+  }
+}
+
 // SILU(gate) * up (src/ops_cpu.cpp:134-141, 167-170), quantised to Q8_0_ACT
 // blocks from the interleaved gate/up pairs; one thread per element, 32 lanes
 // to a block. silu(x) = x / (1 +
@@ -521,8 +559,12 @@ int proj(const mi_hip_qwen2* m, const char* w, int64_t row_bytes, int64_t n, int
       p.x = nullptr;
       p.norm_w = nullptr;
       if (act.norm_w) {
-        hipLaunchKernelGGL(mi::norm_q8_kernel, dim3((unsigned)m_cols), dim3(mi::kNormThreads), 0, m->stream,
-                           act.x, k, act.norm_w, m->hp.rms_eps, m->aq, p.a_nb1, (int)k);
+        if (k <= mi::kNormWideMaxE)
+          hipLaunchKernelGGL(mi::norm_q8_8waves_kernel, dim3((unsigned)m_cols), dim3(512), 0, m->stream, act.x, k,
+                             act.norm_w, m->hp.rms_eps, m->aq, p.a_nb1, (int)k);
+        else
+          hipLaunchKernelGGL(mi::norm_q8_kernel, dim3((unsigned)m_cols), dim3(mi::kNormThreads), 0, m->stream,
+                             act.x, k, act.norm_w, m->hp.rms_eps, m->aq, p.a_nb1, (int)k);
         Q2_TRY(hipGetLastError(), "norm launch");
       } else {
         int rc = quantize_cols(m, act.x, k, m_cols, m->aq);
@@ -531,9 +573,9 @@ int proj(const mi_hip_qwen2* m, const char* w, int64_t row_bytes, int64_t n, int
     }
   }
   if (rope) {
-    // the stacked Q/K rows are stored permuted: rotated in the epilogue when
-    // the streaming form runs a single column, else put back in natural order
-    if (p.x && m_cols == 1 && mi::q8_ring_form(p)) {
+    // the stacked Q/K rows are stored permuted: rotated in the epilogue of the
+    // streaming form or of several columns, else put back in natural order
+    if (m_cols > 1 || (p.x && mi::q8_ring_form(p))) {
       p.rope_on = 1;
       p.rope = *rope;
       // the cached rows [0, pos) of this layer's K and V, position-major: a
@@ -612,6 +654,8 @@ int enqueue_forward(mi_hip_qwen2* m, const int32_t* ids_dev, int T, int n_past, 
     re.k_row = static_cast<char*>(kc) + (int64_t)n_past * (int64_t)cnb[2];
     re.v_row = static_cast<char*>(vc) + (int64_t)n_past * (int64_t)cnb[2];
     re.c_s1 = (int64_t)cnb[1];
+    re.c_s2 = (int64_t)cnb[2];
+    re.q_ld = qkv_rows;
     re.pos = n_past;
     re.hd = hd;
     re.n_q = E;
@@ -688,6 +732,8 @@ int enqueue_forward(mi_hip_qwen2* m, const int32_t* ids_dev, int T, int n_past, 
       ea.n_tokens = T;
       ea.head_dim = hd;
       ea.scale = scale;
+      ea.aq = m->aq;
+      ea.aq_ld = E / 32 * 36;
       if (T == 1) {
         // the CUs without a head bring the next matrices into L2 (together
         // with one round of parameter loads per launch 1048 -> 1003 us a token)
@@ -701,7 +747,9 @@ int enqueue_forward(mi_hip_qwen2* m, const int32_t* ids_dev, int T, int n_past, 
       return rc;
     }
     if (timed) Q2_TRY(hipEventRecord(m->ev[2 * l + 1], st), "hipEventRecord");
-    if ((rc = proj(m, w.wo, m->row_e, E, E, {m->ao, nullptr}, T, m->x, E, m->x, E))) return rc;
+    // (the reference-order kernels leave their output as activation blocks)
+    const bool blocks = m->attn_mode == MI_HIP_QWEN2_ATTN_REFERENCE_ORDER;
+    if ((rc = proj(m, w.wo, m->row_e, E, E, {blocks ? nullptr : m->ao, nullptr}, T, m->x, E, m->x, E))) return rc;
     bool swiglued = false;
     if ((rc = proj(m, w.wgu, m->row_e, 2 * (int64_t)F, E, {m->x, w.ffn_norm}, T, m->gu, 2 * (int64_t)F,
                    nullptr, 0, nullptr, nullptr, m->aq, &swiglued)))
