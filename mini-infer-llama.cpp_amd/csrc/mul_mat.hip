@@ -185,7 +185,9 @@ __device__ inline unsigned lds_take(__attribute__((address_space(3))) unsigned* 
 // EPI: the stacked Q/K/V epilogue (rows permuted within heads; RoPE and the
 // K/V append for one column) -- a separate instantiation, so the plain form
 // carries none of it.
-template <int M, bool EPI>
+// NT: nontemporal requests (a separate instantiation too: a branch in the refill
+// costs the short launches of a decode step 0.2 us each).
+template <int M, bool EPI, bool NT>
 __global__ __launch_bounds__(kQ8RingWaves * kWave) void mul_mat_q8_0_ring_kernel(const Q8MulMat p) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) char ring_lds[];
@@ -237,8 +239,14 @@ __global__ __launch_bounds__(kQ8RingWaves * kWave) void mul_mat_q8_0_ring_kernel
       r = make_rsrc(p.w + start, (unsigned)min<int64_t>(8 * p.w_nb1, total - start));
     }
     if (live || issue_dead) {
+      lds_t* const d = slots + s * kQ8Slot;
+      if constexpr (NT) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) dma16(r, slots + s * kQ8Slot + 1024 * i, (unsigned)(1024 * i + 16 * lane));
+        for (int i = 0; i < 8; ++i) dma16_nt(r, d + 1024 * i, (unsigned)(1024 * i + 16 * lane));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dma16(r, d + 1024 * i, (unsigned)(1024 * i + 16 * lane));
+      }
     }
     return live ? g : -1;
   };
@@ -709,13 +717,19 @@ hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) 
   if (p.x && !rows_form) return hipErrorInvalidValue;  // the prologue exists in the streaming form only
   if (rows_form) {
     const bool epi = p.rope_on || p.perm_hd;
-    const auto fn = p.m == 2 ? mul_mat_q8_0_ring_kernel<2, false>
-                    : epi    ? mul_mat_q8_0_ring_kernel<1, true>
-                             : mul_mat_q8_0_ring_kernel<1, false>;
+    // A matrix larger than the L2s together passes through them once: asked for
+    // nontemporally (151936 x 896, 145 MB: 29.0 -> 25.4 us; the 9.3 MB of a gate
+    // and up pair are in L2 by then, where the hint gains nothing).
+    const bool nt = p.n * p.w_nb1 > (int64_t)32 << 20;
+    const auto fn = p.m == 2 ? mul_mat_q8_0_ring_kernel<2, false, true>
+                    : epi    ? mul_mat_q8_0_ring_kernel<1, true, false>
+                    : nt     ? mul_mat_q8_0_ring_kernel<1, false, true>
+                             : mul_mat_q8_0_ring_kernel<1, false, false>;
     static const hipError_t attr = [] {
-      const void* fns[3] = {(const void*)&mul_mat_q8_0_ring_kernel<1, false>,
-                            (const void*)&mul_mat_q8_0_ring_kernel<1, true>,
-                            (const void*)&mul_mat_q8_0_ring_kernel<2, false>};
+      const void* fns[4] = {(const void*)&mul_mat_q8_0_ring_kernel<1, false, false>,
+                            (const void*)&mul_mat_q8_0_ring_kernel<1, false, true>,
+                            (const void*)&mul_mat_q8_0_ring_kernel<1, true, false>,
+                            (const void*)&mul_mat_q8_0_ring_kernel<2, false, true>};
       hipError_t e = hipSuccess;
       for (const void* f : fns)
         if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kQ8RingLdsAll);
