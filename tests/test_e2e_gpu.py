@@ -340,3 +340,68 @@ def test_tiny_model_unquantised_embedding_with_separate_lm_head(tmp_path, embd_t
         got = np.frombuffer(logits, dtype=np.float32).reshape(len(prompt), -1)
         assert np.array_equal(bits(got), bits(want))
         assert m.generate(prompt, 12) == [int(t) for t in r.stdout.split()]
+
+
+def test_wide_model_incremental_prefill_equals_batched_bitwise(tmp_path):
+    # n_embd 1088: a column too wide for the 8-wave norm, and one column too
+    # wide for the streaming products, so that one-token steps rotate and append
+    # in a launch of their own while the batched prompt does in its epilogue.
+    cfg = dict(TINY, n_embd=1088, n_head=17, n_head_kv=1, n_ff=160, n_layer=1)
+    path = str(tmp_path / "wide.gguf")
+    gg.write_qwen2_q8_0(path, 23, cfg)
+    prompt = gg.prompt_ids(13, 35, cfg["n_vocab"])
+    with Qwen2(path, n_ctx=64, max_tokens=len(prompt)) as m:
+        m.set_attention(mh.MI_HIP_QWEN2_ATTN_REFERENCE_ORDER)
+        _, batched = m.forward(prompt, n_past=0, last_logits_only=False, want_logits=True)
+        batched = np.frombuffer(batched, dtype=np.float32).reshape(len(prompt), -1)
+        for i, t in enumerate(prompt):
+            _, step = m.forward([t], n_past=i, want_logits=True)
+            assert np.array_equal(bits(batched[i]), bits(np.frombuffer(step, dtype=np.float32))), i
+
+
+def test_norm_equals_serial_sum_bitwise(tmp_path, oracle):
+    # One layer whose output and down projections are zero, so that the logits
+    # are lm_head . Q8_0(RMS_NORM(embedding)): against a norm whose squares are
+    # summed one by one in float32, for ordinary rows and for one of equal
+    # values, whose sum drifts out of the 8-wave sum's candidates.
+    seed, tok = 31, 5
+    cfg = dict(TINY, n_layer=1, embd_type=gg.T_F32)
+    path = str(tmp_path / "norm.gguf")
+    gg.write_qwen2_q8_0(path, seed, cfg)
+    data = bytearray(open(path, "rb").read())
+    span, off = {}, 0
+    for name, ne, t, _ in gg.tensor_plan(cfg):
+        n = int(np.prod(ne))
+        size = {gg.T_F32: 4 * n, gg.T_Q8_0: n // 32 * 34}[t]
+        span[name] = (off, size)
+        off += -(-size // gg.GGUF_ALIGN) * gg.GGUF_ALIGN
+    base = len(data) - off
+
+    def view(name):
+        return slice(base + span[name][0], base + sum(span[name]))
+
+    for name in ("blk.0.attn_output.weight", "blk.0.ffn_down.weight"):
+        data[view(name)] = bytes(span[name][1])
+    E, V = cfg["n_embd"], cfg["n_vocab"]
+    embd = np.frombuffer(bytes(data[view("token_embd.weight")]), dtype=np.float32).reshape(V, E).copy()
+    embd[tok] = 3.7
+    data[view("token_embd.weight")] = embd.tobytes()
+    with open(path, "wb") as f:
+        f.write(bytes(data))
+    prompt = [tok, 17, tok, 3]
+    want = []
+    for t in prompt:
+        s = np.float32(0)
+        for v in embd[t]:
+            s = np.float32(s + np.float32(v * v))
+        mean = np.float32(np.float64(s) / np.float64(E))
+        root = np.float32(np.sqrt(np.float64(np.float32(mean + np.float32(cfg["rms_eps"])))))
+        y = embd[t] * np.float32(1.0 / np.float64(root))
+        act = oracle.quantize_q8_0_act(y.reshape(1, E))
+        w = np.frombuffer(bytes(data[view("output.weight")]), dtype=np.uint8)
+        want.append(oracle.mul_mat_q8_0(w, act, E, V, 1)[0])
+    with Qwen2(path, n_ctx=64, max_tokens=len(prompt)) as m:
+        _, batched = m.forward(prompt, n_past=0, last_logits_only=False, want_logits=True)
+        assert np.array_equal(bits(np.frombuffer(batched, dtype=np.float32)), bits(np.concatenate(want)))
+        _, step = m.forward(prompt[:1], n_past=0, want_logits=True)
+        assert np.array_equal(bits(np.frombuffer(step, dtype=np.float32)), bits(want[0]))
