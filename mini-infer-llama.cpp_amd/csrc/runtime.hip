@@ -177,7 +177,7 @@ struct DecodePlan {
   int n_wg = 0;    // workgroups with work (records)
   int grid_x = 0;  // the widest item's workgroups (grid rows are items)
   bool dyn = false;     // dynamic sub-tile claims
-  bool long_waves = false;  // every wave streams 4 or more sub-tiles on average
+  bool long_waves = false;  // every wave streams 3 or more sub-tiles on average (streaming: stream_min)
   bool mf = false;      // matrix-core kernel
   bool stream = false;  // the streaming kernel (decode_stream.hip)
 };
@@ -255,7 +255,7 @@ void plan_items(DecodePlan& p, mi::DecodeItem* it, int n_items, int gpi, int wav
   }
   for (int i = 0; i < n_items; ++i) p.grid_x = std::max(p.grid_x, gpi * it[i].kpg);
   p.n_wg = (int)wg;
-  p.long_waves = sub >= 4 * wg * waves;
+  p.long_waves = sub >= 3 * wg * waves;
 }
 
 // max_groups: the workspace's group capacity (a head split must fit in it).
@@ -295,12 +295,15 @@ DecodePlan plan_decode(mi::DecodeItem* it, int n_items, int n_head_kv, int n_rep
       bool keep = true;
       for (int i = 0; i < n_items; ++i) keep = keep && it[i].kpg >= kpg0[i];
       // An F16 cache takes the split (vector units) only where the split
-      // launch's waves stream fewer than 4 sub-tiles each on average; longer
-      // streams run faster whole on the matrix cores. One layer, F16, with the
-      // split's sub-tiles per wave: 28/4 heads, D 128 at n_kv 8192 (4) 10.7
-      // against 14.5 us split; 14/2 heads, D 64 at 32768 (4) 11.9 against
-      // 14.3; at 8192 (2) 9.5 against 9.6; at 1024-4096 (1) 7.9-8.0 against
-      // 9.0-9.1 split; 28/4 heads at 512 (1) 8.8 against 10.5 split.
+      // launch's waves stream fewer than 3 sub-tiles each on average; longer
+      // streams run faster whole on the matrix cores. F16, with the split's
+      // sub-tiles per wave (a row one tile short of a round number is as long as
+      // the round one: the line is not at 4): 28/4 heads, D 128, one layer at
+      // n_kv 8192 (4) 10.7 us against 14.5 split, at 8147 (3.98) 10.7 against
+      // 14.4; 14/2 heads, D 64, 4 layers at 8147 (3.98) 10.5 against 14.0; 28/4
+      // heads, 4 layers at 2000 (3.9) 13.1 against 14.5, at 1000 (1.96) 11.7
+      // against 10.9; 14/2 heads, one layer at 1000-4096 (1) 8.6-9.0 against
+      // 7.1-7.4, 28/4 heads at 512 (1) 10.9 against 8.5.
       if (autom && f16 && q.long_waves) keep = false;
       if (keep) {
         q.mf = p.mf;  // sub-tiles and workgroups both double: long_waves stands
