@@ -142,7 +142,7 @@ __device__ __forceinline__ void store_out(const ExactAttn& p, int j, int h, int 
 // 1 KB requests; 16-byte slots XOR-swizzled by row if SW, so that one row per
 // lane reads free of bank conflicts. A wave's requests are NW / 4 x 64 / D x 16
 // rows apart, where the swizzle repeats: an address is the one before plus a
-// constant.
+// constant (a computed one cost 20 instructions a request).
 template <int D, int NW, bool SW>
 __device__ __forceinline__ void rows_to_lds(lds_t* dst, const char* base, int64_t s2, int row0, int n, int last,
                                             int w, int lane) {
@@ -176,10 +176,10 @@ __device__ __forceinline__ void rows_to_lds(lds_t* dst, const char* base, int64_
 //
 // Measured (14 / 2 heads, D 64, us per launch; before: one kernel with the
 // whole row in LDS up to 512 keys and one of a wave per row beyond): n_kv 129
-// 7.3 -> 6.7, 301 10.2 -> 8.0, 1501 75.8 -> 22.8. Of the 22.8 the output
-// chains take 10.5 (7 ns a key, 4.2 of them the addition itself), the scores
-// 6.7 (LDS-direct requests bring about 55 GB/s into a CU, and a row has one
-// CU), the exponentials and their sum 2.7.
+// 7.3 -> 6.7, 301 10.2 -> 8.0, 1501 75.4 -> 24.5. There the output chains take
+// 10.5 (7 ns a key, 4.2 of them the addition itself), the scores 6.7
+// (LDS-direct requests bring about 55 GB/s into a CU, and a row has one CU),
+// the exponentials and their sum 2.7.
 constexpr int kRowThreads = 512;
 constexpr int kRowWaves = kRowThreads / kWave;
 constexpr int kRowLoaders = 4;          // waves that form the products
@@ -618,7 +618,7 @@ template <int D>
 static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
   const int n_kv = p.n_past + p.n_tokens;
   const int64_t rows = (int64_t)p.n_tokens * p.n_head;
-  // Rows that get a CU each take a workgroup each (14 rows of 1501 keys: 22.8
+  // Rows that get a CU each take a workgroup each (14 rows of 1501 keys: 24.5
   // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.9 us, 41 a row
   // per workgroup), unless their scores do not fit in LDS (about 4000 keys).
   if (rows <= n_cu || tile_lds_bytes<D, kTileWaves, kTileRows>(n_kv) > kLdsMax) return launch_row<D>(p, n_cu, stream);
