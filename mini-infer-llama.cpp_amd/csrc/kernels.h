@@ -170,7 +170,7 @@ bool q8_ring_form(const Q8MulMat& p);
 bool q8_swiglu_out_ok(const Q8MulMat& p, int n_cu);
 hipError_t launch_quantize_q8_0_act(const Q8Quantize& p, hipStream_t stream);
 hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream);
-// mul_mat_cols.hip: several columns (Q8_0_ACT blocks at p.a, no prologue or SwiGLU).
+// mul_mat_cols.hip: several columns (k > 0, Q8_0_ACT blocks at p.a, no prologue or SwiGLU).
 hipError_t launch_mul_mat_q8_0_cols(const Q8MulMat& p, int n_cu, hipStream_t stream);
 
 // Cache append: src F32 [head_dim, n_head_kv, n_tokens] (device, byte strides)

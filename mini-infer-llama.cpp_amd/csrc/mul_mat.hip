@@ -122,6 +122,17 @@ __global__ __launch_bounds__(256) void mul_mat_q8_0_kernel(const Q8MulMat p) {
   }
 }
 
+// k = 0: every sum is empty, so an output is +0.0 (plus the added term). There
+// is no block to read, and the other kernels read a row's last one.
+__global__ __launch_bounds__(256) void mul_mat_q8_0_empty_kernel(const Q8MulMat p) {
+  const int64_t total = p.n * p.m, step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += step) {
+    const int64_t col = i / p.n, row = i - col * p.n;
+    const float s = p.add ? 0.0f + gload<float>(p.add + row * p.add_nb0 + col * p.add_nb1) : 0.0f;
+    gstore<float>(p.dst + row * p.dst_nb0 + col * p.dst_nb1, s);
+  }
+}
+
 // The streaming form, for weight rows of at most 1 KB (k <= 960: every matrix
 // of a 896-wide model), 16-byte aligned groups of 8 rows and one column (or
 // two of a very tall matrix: q8_ring_form). One workgroup of 8 waves per CU; each wave walks row groups (8
@@ -713,6 +724,13 @@ bool q8_ring_form(const Q8MulMat& p) {
 
 hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) {
   if (p.n == 0 || p.m == 0) return hipSuccess;
+  if (p.k == 0) {
+    if (p.x || p.rope_on || p.perm_hd || p.swiglu_out) return hipErrorInvalidValue;
+    const int64_t groups = (p.n * p.m + 255) / 256;  // (a grid of any size covers the outputs)
+    hipLaunchKernelGGL(mul_mat_q8_0_empty_kernel, dim3((unsigned)std::min<int64_t>(groups, 4096)), dim3(256), 0,
+                       stream, p);
+    return hipGetLastError();
+  }
   const bool rows_form = q8_ring_form(p);
   if (p.x && !rows_form) return hipErrorInvalidValue;  // the prologue exists in the streaming form only
   if (rows_form) {

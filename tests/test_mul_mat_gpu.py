@@ -162,3 +162,20 @@ def test_q8_0_columns_bitwise(hip, stream, oracle, k, n, m):
         hip.check(hip.mi_hip_op_mul_mat(ctypes.byref(d), stream))
         torch.cuda.synchronize()
         assert np.array_equal(bits(got[j]), bits(one.cpu().numpy())), j
+
+
+@pytest.mark.parametrize("n,m", [(1, 1), (75, 1), (40, 2), (33, 17), (1203, 2000)])
+def test_q8_0_no_blocks_gives_zeros(hip, stream, n, m):
+    # k = 0: every dot product is empty. The operands have no block to read:
+    # they point into a buffer of NaN scales, which any read would pull in.
+    import torch
+    poison = torch.full((4096,), 0x7f, dtype=torch.uint8, device="cuda")
+    out = torch.full((m, n + 3), float("nan"), device="cuda")
+    wt = make_tensor(poison.data_ptr() + 2048, [0, n], [34, 0], type_=mh.MI_TYPE_Q8_0)
+    at = make_tensor(poison.data_ptr() + 1024, [0, m], [36, 0], type_=mh.MI_TYPE_Q8_0_ACT)
+    d = make_tensor(out.data_ptr(), [n, m], [4, 4 * (n + 3)], op=mh.MI_OP_MUL_MAT, src=[wt, at])
+    hip.check(hip.mi_hip_op_mul_mat(ctypes.byref(d), stream))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert not bits(got[:, :n]).any()  # +0.0
+    assert np.isnan(got[:, n:]).all()
