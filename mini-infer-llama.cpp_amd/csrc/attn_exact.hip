@@ -302,6 +302,9 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
         request(k0 + 2 * KB, s, KB);
       }
     }
+    // the last requests are past the row, but they are writes all the same:
+    // the products overwrite their buffers
+    wait_vmem<0>();
   }
   if (tid < 32) lds_store<uint64_t>(tab + 8 * tid, te);
   // the first V rows meanwhile, in the loaders' registers, two buffers ahead

@@ -124,6 +124,8 @@ def test_random_shapes_bit_for_bit(hip, stream, case):
     (2, 7, 64, 8200, 1),     # one row per workgroup: half-size K buffers (past 7,000 keys)
     (1, 2, 64, 24500, 1),    # and the smallest ones
     (2, 2, 128, 513, 2),     # a buffer more than both hold at head_dim 128
+    (1, 3, 128, 8200, 1),    # head_dim 128: half-size buffers
+    (1, 2, 128, 24500, 1),   # and the smallest, whose last requests are past the row
     (1, 1, 64, 0, 300),      # more rows than workgroups: tiles, from one key up
     (2, 7, 64, 63, 37),      # key counts across a tile's edge, rows past the last
     (3, 5, 128, 60, 20),     # head_dim 128, 100 rows per KV head
