@@ -277,7 +277,10 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
     request(0, 0, min(n, KB));
     if (n > KB) request(KB, 1, n - KB);
     // V is asked for only after the scores: a dword of each of its 128-byte
-    // lines now, so that they are in L2 by then
+    // lines now, so that they are in L2 by then. The wait below counts these
+    // loads as the wave's latest: the fence keeps them behind the requests
+    // (and the wait, which clobbers memory too, keeps them before it).
+    asm volatile("" ::: "memory");
     constexpr int kLines = D / 32, kTouch = (2 * KB * kLines + kRowThreads - 1) / kRowThreads;
     unsigned vt[kTouch];
 #pragma unroll
