@@ -11,10 +11,12 @@
 //
 // The order leaves two chains of a dependent additions per row (8.4 cycles
 // each: 3.5 ns), the sum of the exponentials and an output element's sum;
-// everything else is independent and is taken off them. Few rows (a decode
-// step) run one workgroup per row, which shortens the chains
-// (attn_exact_row_kernel); many rows (a prompt) run several rows per wave,
-// which share the K and V tiles and fill the chip (attn_exact_tile_kernel).
+// everything else is independent and is taken off them. Short rows run one
+// workgroup per row with all its K, then V rows in LDS
+// (attn_exact_staged_kernel); few longer rows (a decode step) one workgroup
+// per row that shortens the chains (attn_exact_row_kernel); many (a prompt) one
+// row per wave, whose workgroups share the K and V tiles and fill the chip
+// (attn_exact_tile_kernel).
 #include <algorithm>
 #include <cmath>
 
@@ -141,31 +143,232 @@ __device__ __forceinline__ void store_out(const ExactAttn& p, int j, int h, int 
 // LDS, n * D / 4 a multiple of 64, by NW waves of which this is the w-th: whole
 // 1 KB requests; 16-byte slots XOR-swizzled by row if SW, so that one row per
 // lane reads free of bank conflicts. A wave's requests are NW / 4 x 64 / D x 16
-// rows apart, where the swizzle repeats: an address is the one before plus a
-// constant (a computed one cost 20 instructions a request).
+// rows apart: an address is the one before plus a constant (a computed one
+// cost 20 instructions a request), but for the slot where the swizzle does not
+// repeat.
 template <int D, int NW, bool SW>
 __device__ __forceinline__ void rows_to_lds(lds_t* dst, const char* base, int64_t s2, int row0, int n, int last,
                                             int w, int lane) {
   constexpr int PPR = D / 4;  // 16-byte pieces per row
   constexpr int STEP = kWave * NW / PPR;
-  static_assert(!SW || STEP % 16 == 0, "the swizzle repeats every 16 rows");
-  const int r = (kWave * w + lane) / PPR, slot = lane % PPR;
-  const int col = 16 * (SW ? slot ^ swz<PPR>(r) : slot);
+  const int slot = lane % PPR;
+  int r = (kWave * w + lane) / PPR;
+  int col = 16 * (SW ? slot ^ swz<PPR>(r) : slot);
+  auto next = [&]() __attribute__((always_inline)) {
+    r += STEP;
+    if (SW && STEP % 16 != 0) col = 16 * (slot ^ swz<PPR>(r));
+  };
   if (row0 + n - 1 <= last) {
-    const char* p = base + (int64_t)(row0 + r) * s2 + col;
+    const char* p = base + (int64_t)(row0 + r) * s2;
     for (int i0 = kWave * w; i0 < n * PPR; i0 += kWave * NW) {
-      dma16_from(p, dst + 16 * i0);
+      dma16_from(p + col, dst + 16 * i0);
       p += STEP * s2;
+      next();
     }
   } else {
-    for (int i0 = kWave * w, q = row0 + r; i0 < n * PPR; i0 += kWave * NW, q += STEP)
-      dma16_from(base + (int64_t)min(q, last) * s2 + col, dst + 16 * i0);
+    for (int i0 = kWave * w; i0 < n * PPR; i0 += kWave * NW) {
+      dma16_from(base + (int64_t)min(row0 + r, last) * s2 + col, dst + 16 * i0);
+      next();
+    }
+  }
+}
+
+// A workgroup past the rows: its share of what the next launches read, pieces
+// of its own XCD (the same workgroup number modulo 8).
+template <int T>
+__device__ __forceinline__ void warm_up(const ExactAttn& p) {
+  const int n_rows = p.n_tokens * p.n_head;
+  const int xcd = blockIdx.x % 8, first = (n_rows + 7 - xcd) / 8, per_xcd = ((int)gridDim.x + 7 - xcd) / 8 - first;
+  for (int w = 0, c = blockIdx.x / 8 - first; w < kMaxWarmUps; ++w) {
+    const int n = (p.warm[w].n + 7 - xcd) / 8;  // pieces of this XCD
+    for (; c < n; c += per_xcd)
+      warm_lines(p.warm[w].p + (int64_t)(xcd + 8 * c) * p.warm[w].bytes, p.warm[w].bytes, threadIdx.x, T);
+    c -= n;
   }
 }
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// One workgroup per (token, head).
+// One workgroup of 4 waves per (token, head), for short rows: all K rows come
+// into LDS and the threads form one key's score each from there; then three
+// waves bring the V rows over the K rows while wave 0 forms the maximum, the
+// exponentials and their ordered sum; then each output element's lane runs its
+// ordered V sum from LDS. Fewer barriers than the kernel below and nothing to
+// divide, which is what short rows take their time for (a launch takes 3.4 us
+// with 16 keys, where the row kernel takes 5.3), at the price of LDS for a
+// whole row's V and of the sums' whole chains (7 ns a key and chain).
+constexpr int kStagedThreads = 256;
+constexpr int kStagedWaves = kStagedThreads / kWave;
+
+// The V rows (whole 1 KB requests) and the probabilities have 16 entries of
+// room past n_kv: the ordered sums read the chunk past the last whole one too.
+__host__ __device__ inline int staged_v_bytes(int n_kv, int d) { return ((n_kv + 16) * d * 4 + 1023) & ~1023; }
+__host__ __device__ inline int staged_prob_bytes(int n_kv) { return 4 * (((n_kv + 15) & ~15) + 16); }
+inline int staged_lds_bytes(int n_kv, int d) { return staged_v_bytes(n_kv, d) + staged_prob_bytes(n_kv) + 256 + 32; }
+
+// acc + v[0] * p[0] + v[D] * p[1] + ... + v[(n - 1) D] * p[n - 1], each
+// product and sum rounded (v: one output element's column of V rows D floats
+// apart; 16 rows and probabilities readable past n). The products do not
+// depend on the running sum: chunk c + 1's 16 are formed between chunk c's
+// additions, so each addition waits only for the one before it, not for a
+// multiplication issued just before it. (The same products, added in the
+// same order: the same bits.)
+template <int D>
+__device__ __forceinline__ float exact_dot(const lds_t* v, const lds_t* p, int n) {
+#pragma clang fp contract(off)
+  float acc = 0.0f;
+  float va[16], vb[16];
+  f32x4_t pa[4], pb[4];
+  float ra[16], rb[16];  // products
+  auto get = [&](float (&vv)[16], f32x4_t (&pp)[4], int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) vv[u] = lds_load<float>(v + 4 * D * (16 * c + u));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) pp[u] = lds_load<f32x4_t>(p + 64 * c + 16 * u);
+  };
+  auto prod = [&](float (&r)[16], const float (&vv)[16], const f32x4_t (&pp)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      r[4 * u] = vv[4 * u] * pp[u].x;
+      r[4 * u + 1] = vv[4 * u + 1] * pp[u].y;
+      r[4 * u + 2] = vv[4 * u + 2] * pp[u].z;
+      r[4 * u + 3] = vv[4 * u + 3] * pp[u].w;
+    }
+  };
+  // chunk r's additions, chunk (vv, pp)'s products into rn between them
+  auto add_prod = [&](const float (&r)[16], float (&rn)[16], const float (&vv)[16], const f32x4_t (&pp)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      acc = acc + r[4 * u];
+      rn[4 * u] = vv[4 * u] * pp[u].x;
+      acc = acc + r[4 * u + 1];
+      rn[4 * u + 1] = vv[4 * u + 1] * pp[u].y;
+      acc = acc + r[4 * u + 2];
+      rn[4 * u + 2] = vv[4 * u + 2] * pp[u].z;
+      acc = acc + r[4 * u + 3];
+      rn[4 * u + 3] = vv[4 * u + 3] * pp[u].w;
+    }
+  };
+  auto add = [&](const float (&r)[16]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 16; ++t) acc = acc + r[t];
+  };
+  const int nch = n >> 4;
+  if (nch > 0) {
+    get(va, pa, 0);
+    prod(ra, va, pa);
+    if (nch > 1) get(vb, pb, 1);
+    int c = 0;
+    // ra: chunk c's products; vb, pb: chunk c + 1's values
+    for (; c + 2 < nch; c += 2) {
+      get(va, pa, c + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      add_prod(ra, rb, vb, pb);
+      get(vb, pb, c + 3);  // (c + 3 <= nch: at most the chunk past the last whole one)
+      __builtin_amdgcn_sched_barrier(0);
+      add_prod(rb, ra, va, pa);
+    }
+    if (c + 1 < nch) {
+      add_prod(ra, rb, vb, pb);
+      add(rb);
+    } else {
+      add(ra);
+    }
+  }
+  for (int t = 16 * nch; t < n; ++t) acc = acc + lds_load<float>(v + 4 * D * t) * lds_load<float>(p + 4 * t);
+  return acc;
+}
+
+template <int D>
+__global__ __launch_bounds__(kStagedThreads) void attn_exact_staged_kernel(const ExactAttn p) {
+#pragma clang fp contract(off)
+  extern __shared__ __attribute__((aligned(16))) char ex_lds[];
+  lds_t* const lds = (lds_t*)ex_lds;
+  constexpr int PPR = D / 4;               // 16-byte pieces per row
+  constexpr int kWhole = kWave / PPR;      // rows per request
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // every parameter in one round of scalar loads, not one where each is first used
+  asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.q_s1), "s"(p.q_s2), "s"(p.k_s1), "s"(p.k_s2), "s"(p.v_s1),
+               "s"(p.v_s2), "s"(p.n_head), "s"(p.n_rep), "s"(p.n_past), "s"(p.n_tokens), "s"(p.scale), "s"(p.out),
+               "s"(p.o_s1), "s"(p.o_s2), "s"(p.aq), "s"(p.aq_ld));
+  if ((int)blockIdx.x >= p.n_tokens * p.n_head) {
+    warm_up<kStagedThreads>(p);
+    return;
+  }
+  const int h = blockIdx.x % p.n_head;
+  const int j = p.n_tokens - 1 - blockIdx.x / p.n_head;  // the longest rows first
+  const int kvh = h / p.n_rep;
+  const int a = p.n_past + j + 1, n_kv = p.n_past + p.n_tokens;
+  lds_t* const rows = lds;  // K, later V
+  lds_t* const prob = lds + staged_v_bytes(n_kv, D);
+  lds_t* const tab = prob + staged_prob_bytes(n_kv);
+  lds_t* const red = tab + 256;
+  const uint64_t te = kExpfTab[lane & 31];  // requested first: loads complete in order
+  const int n_req = (a + kWhole - 1) & ~(kWhole - 1);  // rows requested
+  rows_to_lds<D, kStagedWaves, true>(rows, p.k + kvh * p.k_s1, p.k_s2, 0, n_req, a - 1, wv, lane);
+  // the query meanwhile (a uniform address: scalar loads)
+  const char* q = p.q + h * p.q_s1 + (int64_t)j * p.q_s2;
+  f32x4_t qv[PPR];
+#pragma unroll
+  for (int u = 0; u < PPR; ++u) qv[u] = *(const __attribute__((address_space(4))) f32x4_t*)(q + 16 * u);
+  wait_vmem<0>();  // this wave's K requests have landed
+  wg_barrier();
+  // one key's score per thread, d ascending, product and sum each rounded
+  float mx = -INFINITY;
+  for (int i = tid; i < a; i += kStagedThreads) {
+    const lds_t* const rowp = rows + i * (4 * D);
+    // the D products first (independent), then their sum in order
+    float pr[D];
+#pragma unroll
+    for (int u = 0; u < PPR; ++u) {
+      const f32x4_t kv = lds_load<f32x4_t>(rowp + 16 * (u ^ swz<PPR>(i)));
+      pr[4 * u] = kv.x * qv[u].x;
+      pr[4 * u + 1] = kv.y * qv[u].y;
+      pr[4 * u + 2] = kv.z * qv[u].z;
+      pr[4 * u + 3] = kv.w * qv[u].w;
+    }
+    float acc = 0.0f;
+#pragma unroll
+    for (int d = 0; d < D; ++d) acc = acc + pr[d];
+    const float v = acc * p.scale;
+    lds_store<float>(prob + 4 * i, v);
+    mx = v > mx ? v : mx;
+  }
+  mx = wave_max_dpp(mx);  // (never NaN; the sign of a zero maximum changes no exponential)
+  if (tid < 32) lds_store<uint64_t>(tab + 8 * tid, te);
+  if (lane == 0) lds_store<float>(red + 4 * wv, mx);
+  wg_barrier();  // the scores are in LDS and every K row has been read
+  if (wv > 0) {
+    rows_to_lds<D, kStagedWaves - 1, false>(rows, p.v + kvh * p.v_s1, p.v_s2, 0, n_req, a - 1, wv - 1, lane);
+    wait_vmem<0>();  // this wave's V requests have landed
+  } else {
+    mx = lds_load<float>(red);
+#pragma unroll
+    for (int w = 1; w < kStagedWaves; ++w) {
+      const float o = lds_load<float>(red + 4 * w);
+      mx = o > mx ? o : mx;
+    }
+    // zeros past the keys, up to a whole chunk: they leave the sum unchanged
+    const int n_pad = (a + 15) & ~15;
+    for (int i = lane; i < n_pad; i += kWave) {
+      const float x = lds_load<float>(prob + 4 * i) - mx;
+      lds_store<float>(prob + 4 * i,
+                       i < a ? expf_ref(x, (const __attribute__((address_space(3))) uint64_t*)tab) : 0.0f);
+    }
+    wave_lds_fence();
+    const float sum = exact_sum(prob, n_pad, 0.0f);
+    if (lane == 0) lds_store<float>(red + 16, (float)(1.0 / (double)sum));  // the correctly rounded 1.0f / sum
+  }
+  wg_barrier();  // the V rows and 1 / sum
+  const float inv = lds_load<float>(red + 16);
+  for (int i = tid; i < a; i += kStagedThreads) lds_store<float>(prob + 4 * i, lds_load<float>(prob + 4 * i) * inv);
+  wg_barrier();
+  if (tid < D) store_out(p, j, h, tid, exact_dot<D>(rows + 4 * tid, prob, a));
+}
+
+// ---------------------------------------------------------------------------
+// One workgroup per (token, head), for longer rows.
 //
 // Scores: K rows come through two LDS buffers, one key per thread. The sum of
 // the exponentials is cut into 8 segments, one per wave, run from 64 candidate
@@ -209,17 +412,8 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
   // every parameter in one round of scalar loads, not one where each is first used
   asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.q_s1), "s"(p.q_s2), "s"(p.k_s1), "s"(p.k_s2), "s"(p.v_s1),
                "s"(p.v_s2), "s"(p.n_head), "s"(p.n_rep), "s"(p.n_past), "s"(p.n_tokens), "s"(p.scale));
-  const int n_rows = p.n_tokens * p.n_head;
-  if ((int)blockIdx.x >= n_rows) {
-    // a workgroup past the rows: its share of what the next launches read,
-    // pieces of its own XCD (the same workgroup number modulo 8)
-    const int xcd = blockIdx.x % 8, first = (n_rows + 7 - xcd) / 8, per_xcd = ((int)gridDim.x + 7 - xcd) / 8 - first;
-    for (int w = 0, c = blockIdx.x / 8 - first; w < kMaxWarmUps; ++w) {
-      const int n = (p.warm[w].n + 7 - xcd) / 8;  // pieces of this XCD
-      for (; c < n; c += per_xcd)
-        warm_lines(p.warm[w].p + (int64_t)(xcd + 8 * c) * p.warm[w].bytes, p.warm[w].bytes, tid, kRowThreads);
-      c -= n;
-    }
+  if ((int)blockIdx.x >= p.n_tokens * p.n_head) {
+    warm_up<kRowThreads>(p);
     return;
   }
   const int h = blockIdx.x % p.n_head;
@@ -578,17 +772,32 @@ __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAt
   }
 }
 
+// Workgroups past the rows: what is to be warmed up gets the idle CUs, two
+// pieces each.
+static int side_workgroups(const ExactAttn& p, int n_cu) {
+  int64_t pieces = 0;
+  for (const WarmUp& w : p.warm) pieces += w.n;
+  return (int)std::min<int64_t>(std::max(n_cu - p.n_tokens * p.n_head, 0) & ~7, (pieces + 15) / 16 * 8);
+}
+
+template <int D>
+static hipError_t launch_staged(const ExactAttn& p, int n_cu, hipStream_t stream) {
+  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_staged_kernel<D>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
+  if (attr != hipSuccess) return attr;
+  const int rows = p.n_tokens * p.n_head;
+  hipLaunchKernelGGL(attn_exact_staged_kernel<D>, dim3((unsigned)(rows + side_workgroups(p, n_cu))),
+                     dim3(kStagedThreads), (unsigned)staged_lds_bytes(p.n_past + p.n_tokens, D), stream, p);
+  return hipGetLastError();
+}
+
 template <int D, int BUF, int CK>
 static hipError_t launch_row(const ExactAttn& p, int n_cu, hipStream_t stream) {
   static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_row_kernel<D, BUF, CK>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
   if (attr != hipSuccess) return attr;
-  // what is to be warmed up gets the idle CUs, two pieces each
   const int rows = p.n_tokens * p.n_head;
-  int64_t pieces = 0;
-  for (const WarmUp& w : p.warm) pieces += w.n;
-  const int side = (int)std::min<int64_t>(std::max(n_cu - rows, 0) & ~7, (pieces + 15) / 16 * 8);
-  hipLaunchKernelGGL((attn_exact_row_kernel<D, BUF, CK>), dim3((unsigned)(rows + side)), dim3(kRowThreads),
+  hipLaunchKernelGGL((attn_exact_row_kernel<D, BUF, CK>), dim3((unsigned)(rows + side_workgroups(p, n_cu))), dim3(kRowThreads),
                      (unsigned)row_lds_bytes(p.n_past + p.n_tokens, BUF), stream, p);
   return hipGetLastError();
 }
@@ -620,10 +829,25 @@ static hipError_t launch_tile(const ExactAttn& p, hipStream_t stream) {
 // with 8 of 2, 8.3 with 4 of 1; 384 tokens 20.1, 23.8 and 19.5.
 constexpr int kTileWaves = 8, kTileRows = 1;
 
+// Short rows: as many as run at once (LDS, and 5 or 3 waves' registers per
+// SIMD) and, where every row has a CU, up to the length at which the row kernel
+// overtakes. us, staged against row or tile: 1 row x 14 heads of 64, n_kv 16
+// 3.4 / 5.3, 128 4.9 / 6.3, 256 6.8 / 7.7, 301 8.7 / 8.5; 28 heads of 128, 257
+// 10.3 / 14.4 (301 no longer fits). Heads of 64, 19 rows after 256 8.6 / 13.4,
+// 64 after 40 5.8 / 7.2, 96 after 40 (more than run at once) 9.4 / 8.8; of 128,
+// 24 after 0 5.2 / 5.8, 32 after 0 7.8 / 6.0.
+template <int D>
+static bool staged_form(int n_kv, int64_t rows, int n_cu) {
+  const int per_cu = kLdsMax / staged_lds_bytes(n_kv, D);
+  if (rows <= n_cu) return D == 64 ? n_kv <= 256 : per_cu > 0;
+  return rows <= (int64_t)n_cu * std::min(per_cu, D == 64 ? 4 : 3);
+}
+
 template <int D>
 static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
   const int n_kv = p.n_past + p.n_tokens;
   const int64_t rows = (int64_t)p.n_tokens * p.n_head;
+  if (staged_form<D>(n_kv, rows, n_cu)) return launch_staged<D>(p, n_cu, stream);
   // Rows that get a CU each take a workgroup each (14 rows of 1501 keys: 24.5
   // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.9 us, 41 a row
   // per workgroup), unless their scores do not fit in LDS (about 4000 keys).

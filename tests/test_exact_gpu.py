@@ -2,10 +2,11 @@
 the reference's own operation order (src/ops_cpu.cpp:304-410), against the
 oracle (the same order, the host C library's expf) BIT FOR BIT.
 
-Rows of up to 512 keys at head_dim 64 (256 at 128) run the staged kernel (V
-rows in LDS, the ordered sums read in chunks of 16 ahead of their additions);
-longer rows run the unstaged kernel. Key counts cover one key, partial and
-whole chunks of 16, odd and even chunk counts, the staged limit and past it,
+Short rows run the staged kernel (K, then V rows in LDS; up to 256 keys at
+head_dim 64, as many as fit at 128, and only as many rows as run at once), few
+longer rows the row kernel (a workgroup per row), many the tile kernel (a row
+per wave). Key counts cover one key, partial and whole chunks of 16, odd and
+even chunk counts, the staged limit and past it,
 prefill rows on both sides of it, and a row whose exponentials are all equal
 but one (its one-lane sum rounds the same way step after step). 32 seeded
 random shapes (1-8 KV heads, 1-8 Q heads each, decode rows and short
@@ -55,7 +56,7 @@ def _check(hip, stream, q, k, v, n_past, scale, what):
 
 @pytest.mark.parametrize("d,n_kv", [(64, 1), (64, 15), (64, 16), (64, 17), (64, 33), (64, 129), (64, 256),
                                     (64, 383), (64, 512), (64, 513), (64, 1000), (128, 31), (128, 255),
-                                    (128, 256), (128, 257)])
+                                    (128, 256), (128, 257), (128, 300), (128, 301)])
 def test_decode_bit_for_bit(hip, stream, d, n_kv):
     q, k, v = _inputs(1000 + n_kv, 1, n_kv, 14, 2, d)
     _check(hip, stream, q, k, v, n_kv - 1, float(np.float32(1) / np.sqrt(np.float32(d))),
@@ -65,7 +66,7 @@ def test_decode_bit_for_bit(hip, stream, d, n_kv):
 @pytest.mark.parametrize("n_tokens,n_past,h,hkv", [(37, 100, 14, 2), (20, 600, 14, 2), (9, 0, 8, 8),
                                                     (16, 481, 28, 4)])
 def test_prefill_rows_bit_for_bit(hip, stream, n_tokens, n_past, h, hkv):
-    # rows of one call span staged and unstaged key counts (n_past + j + 1)
+    # rows of one call span several key counts (n_past + j + 1)
     q, k, v = _inputs(7 + n_past, n_tokens, n_past + n_tokens, h, hkv, 64)
     _check(hip, stream, q, k, v, n_past, 0.125, f"prefill {n_tokens} rows after {n_past}, {h}/{hkv} heads")
 
@@ -97,8 +98,7 @@ def test_rejects_what_it_does_not_cover(hip, stream):
 
 def _random_cases(n, seed):
     # (case, n_head_kv, n_rep, head_dim, n_past, n_tokens, scale): decode rows and
-    # short prefills, key counts spread log-uniformly over 1..3000 (the staged
-    # kernel below 512 keys at head_dim 64 / 256 at 128, the unstaged above)
+    # short prefills, key counts spread log-uniformly over 1..3000
     rng = np.random.default_rng(seed)
     out = []
     for i in range(n):
@@ -127,7 +127,11 @@ def test_random_shapes_bit_for_bit(hip, stream, case):
     (1, 3, 128, 8200, 1),    # head_dim 128: half-size buffers
     (1, 2, 128, 24500, 1),   # and the smallest, whose last requests are past the row
     (1, 1, 64, 0, 300),      # more rows than workgroups: tiles, from one key up
-    (2, 7, 64, 63, 37),      # key counts across a tile's edge, rows past the last
+    (2, 7, 64, 63, 37),      # more rows than workgroups and few keys: staged, several a CU
+    (2, 7, 64, 55, 73),      # 128 keys, and more rows than run at once: tiles
+    (2, 7, 64, 56, 73),      # one key more: across a tile's edge
+    (3, 5, 128, 3, 51),      # head_dim 128: 765 rows staged,
+    (3, 5, 128, 3, 52),      # 780 in tiles, rows past the last
     (3, 5, 128, 60, 20),     # head_dim 128, 100 rows per KV head
     (1, 8, 64, 4300, 40),    # more rows than workgroups, scores too long for tiles
 ])
