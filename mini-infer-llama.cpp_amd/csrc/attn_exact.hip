@@ -393,7 +393,7 @@ constexpr int kLdsMax = 160 * 1024;
 __host__ __device__ inline int row_segment(int n) { return ((n + 7) / 8 + 15) & ~15; }
 __host__ __device__ inline int row_prob_bytes(int n) { return 4 * (8 * row_segment(n) + 16); }
 inline int row_lds_bytes(int n, int buf) { return row_prob_bytes(n) + kRowWork + 2 * buf; }
-static_assert(4 * (kExactMaxKeys + 16) + kRowWork + 2 * 8 * 1024 <= kLdsMax, "the longest row fits");
+static_assert(4 * (kExactMaxKeys + 16) + kRowWork + 2 * 14 * 1024 <= kLdsMax, "the longest row fits");
 
 // BUF: bytes of a buffer of K rows (two, whole requests of every wave), later
 // of CK rows of products.
@@ -404,8 +404,9 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
   lds_t* const lds = (lds_t*)ex_lds;
   constexpr int PPR = D / 4;
   constexpr int KB = BUF / (4 * D);                       // keys per buffer
-  constexpr int kReq = BUF / (1024 * kRowWaves);          // requests per wave and buffer
-  static_assert(kReq * 1024 * kRowWaves == BUF && KB <= kRowThreads, "whole requests, a key per thread");
+  constexpr int kReq = BUF / (1024 * kRowWaves);          // requests per wave and buffer, at least
+  static_assert(BUF % 1024 == 0 && kReq > 0 && KB <= kRowThreads, "whole requests, a key per thread");
+  static_assert(CK % 16 == 0 && 4 * CK * D <= BUF, "whole chunks of products in a buffer");
   constexpr int NV = CK * PPR / (kRowLoaders * kWave);    // pieces of V per loader thread and buffer
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -809,7 +810,10 @@ static hipError_t launch_row(const ExactAttn& p, int n_cu, hipStream_t stream) {
   if (n_kv <= 512) return launch_row<D, 64 * 1024, 4096 / D>(p, n_cu, stream);
   if (row_lds_bytes(n_kv, 64 * 1024) <= kLdsMax) return launch_row<D, 64 * 1024, 8192 / D>(p, n_cu, stream);
   if (row_lds_bytes(n_kv, 32 * 1024) <= kLdsMax) return launch_row<D, 32 * 1024, 8192 / D>(p, n_cu, stream);
-  return launch_row<D, 8 * 1024, 2048 / D>(p, n_cu, stream);
+  // (28 heads of 128, us a launch: 24001 keys 1523, with buffers of 8 KB 2690;
+  // 32001 keys 2040, 3590. From 32129 keys on the buffers are of 14 KB.)
+  if (row_lds_bytes(n_kv, 16 * 1024) <= kLdsMax) return launch_row<D, 16 * 1024, 4096 / D>(p, n_cu, stream);
+  return launch_row<D, 14 * 1024, D == 64 ? 48 : 16>(p, n_cu, stream);
 }
 
 template <int D, int W, int R>

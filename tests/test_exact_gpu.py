@@ -122,10 +122,16 @@ def test_random_shapes_bit_for_bit(hip, stream, case):
 
 @pytest.mark.parametrize("hkv,n_rep,d,n_past,n_tok", [
     (2, 7, 64, 8200, 1),     # one row per workgroup: half-size K buffers (past 7,000 keys)
-    (1, 2, 64, 24500, 1),    # and the smallest ones
+    (1, 2, 64, 24500, 1),    # quarter-size ones
+    (1, 1, 64, 32127, 1),    # the last key count with those
+    (1, 1, 64, 32128, 1),    # and the smallest ones
+    (1, 2, 64, 32767, 1),
     (2, 2, 128, 513, 2),     # a buffer more than both hold at head_dim 128
     (1, 3, 128, 8200, 1),    # head_dim 128: half-size buffers
-    (1, 2, 128, 24500, 1),   # and the smallest, whose last requests are past the row
+    (1, 2, 128, 24500, 1),   # quarter-size ones, whose last requests are past the row
+    (1, 1, 128, 32127, 1),
+    (1, 1, 128, 32128, 1),
+    (1, 2, 128, 32767, 1),
     (1, 1, 64, 0, 300),      # more rows than workgroups: tiles, from one key up
     (2, 7, 64, 63, 37),      # more rows than workgroups and few keys: staged, several a CU
     (2, 7, 64, 55, 73),      # 128 keys, and more rows than run at once: tiles
