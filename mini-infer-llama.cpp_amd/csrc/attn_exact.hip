@@ -16,7 +16,8 @@
 // (attn_exact_staged_kernel); few longer rows (a decode step) one workgroup
 // per row that shortens the chains (attn_exact_row_kernel); many (a prompt) one
 // row per wave, whose workgroups share the K and V tiles and fill the chip
-// (attn_exact_tile_kernel).
+// (attn_exact_tile_kernel); of many rows too long for those, some run one row
+// per wave on its own (attn_exact_wave_kernel).
 #include <algorithm>
 #include <cmath>
 
@@ -773,6 +774,65 @@ __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAt
   }
 }
 
+// ---------------------------------------------------------------------------
+// One wave per (token, head), its probabilities alone in LDS: lanes split the
+// keys, then the output elements, straight from memory. Slow for one row (its
+// chains wait for every read), but a CU holds as many rows as its LDS has room
+// for: see long_form.
+__global__ __launch_bounds__(kWave) void attn_exact_wave_kernel(const ExactAttn p) {
+#pragma clang fp contract(off)
+  extern __shared__ float prob[];
+  __shared__ float s_inv;
+  const int lane = threadIdx.x;
+  const int h = blockIdx.x % p.n_head;
+  const int j = blockIdx.x / p.n_head;
+  const int kvh = h / p.n_rep;
+  const int D = p.head_dim;
+  const int a = min(p.n_past + j + 1, p.n_past + p.n_tokens);
+  const float* q = reinterpret_cast<const float*>(p.q + h * p.q_s1 + (int64_t)j * p.q_s2);
+  float mx = -INFINITY;
+  for (int i = lane; i < a; i += kWave) {
+    const float* kr = reinterpret_cast<const float*>(p.k + kvh * p.k_s1 + (int64_t)i * p.k_s2);
+    float acc = 0.0f;
+#pragma unroll 16  // (the row's loads in flight together)
+    for (int d = 0; d < D; d += 4) {
+      const float4 kv = *reinterpret_cast<const float4*>(kr + d);
+      const float4 qv = *reinterpret_cast<const float4*>(q + d);
+      acc = acc + kv.x * qv.x;
+      acc = acc + kv.y * qv.y;
+      acc = acc + kv.z * qv.z;
+      acc = acc + kv.w * qv.w;
+    }
+    const float v = acc * p.scale;
+    prob[i] = v;
+    mx = v > mx ? v : mx;
+  }
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    const float o = __shfl_xor(mx, off);
+    mx = o > mx ? o : mx;
+  }
+  for (int i = lane; i < a; i += kWave) prob[i] = expf_ref(prob[i] - mx, kExpfTab);
+  __syncthreads();
+  if (lane == 0) {
+    float sum = 0.0f;
+    for (int i = 0; i < a; ++i) sum = sum + prob[i];
+    s_inv = (float)(1.0 / (double)sum);  // the correctly rounded 1.0f / sum
+  }
+  __syncthreads();
+  const float inv = s_inv;
+  for (int i = lane; i < a; i += kWave) prob[i] = prob[i] * inv;
+  __syncthreads();
+  const char* vbase = p.v + kvh * p.v_s1;
+  for (int o = lane; o < D; o += kWave) {
+    float acc = 0.0f;
+#pragma unroll 16  // (16 keys' loads in flight ahead of the ordered additions)
+    for (int t = 0; t < a; ++t)
+      acc = acc + *reinterpret_cast<const float*>(vbase + (int64_t)t * p.v_s2 + 4 * o) * prob[t];
+    store_out(p, j, h, o, acc);
+  }
+}
+
+
 // Workgroups past the rows: what is to be warmed up gets the idle CUs, two
 // pieces each.
 static int side_workgroups(const ExactAttn& p, int n_cu) {
@@ -829,6 +889,40 @@ static hipError_t launch_tile(const ExactAttn& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+static hipError_t launch_wave(const ExactAttn& p, hipStream_t stream) {
+  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_wave_kernel,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kExactMaxKeys * 4);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(attn_exact_wave_kernel, dim3((unsigned)(p.n_tokens * p.n_head)), dim3(kWave),
+                     4 * (unsigned)(p.n_past + p.n_tokens), stream, p);
+  return hipGetLastError();
+}
+
+// Rows whose scores do not fit in LDS eight to a workgroup (about 4000 keys of
+// 64 elements, 3000 of 128), more than there are CUs: the row kernel runs one a
+// CU, tiles of 4 rows run 4 (to 8128 keys, 6080), the wave kernel as many as
+// LDS has room for, each the slower the more they are. What a round of each
+// takes, in ns a key, measured on launches of 20 to 128 tokens x 14 heads of 64
+// and 28 of 128 after 3200 to 16000 keys, which it says the faster form of. us,
+// row / tile / wave: 14 heads of 64, 20 tokens after 4300 113 / 163 / 196, 100
+// (wave) 324 / 319 / 307, 128 (tile) 399 / 328 / 364; 28 of 128, 40 after 4300
+// (tile) 593 / 484 / 533, after 7600 (wave) 1341 / - / 935, after 8200 (row)
+// 1446 / - / 1717.
+enum class LongForm { kRow, kTile, kWave };
+template <int D>
+static LongForm long_form(int n_kv, int64_t rows, int n_cu) {
+  const int64_t per_cu = kLdsMax / (4 * n_kv), whole = rows / (n_cu * per_cu);
+  const double rest = (double)(rows - whole * n_cu * per_cu) / n_cu;
+  auto rounds = [](int64_t n, int64_t at_once) { return (double)((n + at_once - 1) / at_once); };
+  auto wave_round = [](double at_once) { return D == 64 ? 40 + 6 * at_once : 77 + 10 * at_once; };
+  const bool whole_buffers = row_lds_bytes(n_kv, 64 * 1024) <= kLdsMax;
+  const double row = rounds(rows, n_cu) * (D == 64 ? (whole_buffers ? 14 : 15) : (whole_buffers ? 28.5 : 36));
+  const double wave = whole * wave_round((double)per_cu) + (rest > 0 ? wave_round(rest) : 0);
+  const double tile = tile_lds_bytes<D, 4, 1>(n_kv) <= kLdsMax ? rounds(rows, 4 * n_cu) * (D == 64 ? 38 : 57) : row + 1;
+  if (row <= tile && row <= wave) return LongForm::kRow;
+  return tile <= wave ? LongForm::kTile : LongForm::kWave;
+}
+
 // One row per wave: 128 tokens of 14 heads 7.9 us with 8 waves of 1 row, 10.1
 // with 8 of 2, 8.3 with 4 of 1; 384 tokens 20.1, 23.8 and 19.5.
 constexpr int kTileWaves = 8, kTileRows = 1;
@@ -854,9 +948,17 @@ static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
   if (staged_form<D>(n_kv, rows, n_cu)) return launch_staged<D>(p, n_cu, stream);
   // Rows that get a CU each take a workgroup each (14 rows of 1501 keys: 24.5
   // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.9 us, 41 a row
-  // per workgroup), unless their scores do not fit in LDS (about 4000 keys).
-  if (rows <= n_cu || tile_lds_bytes<D, kTileWaves, kTileRows>(n_kv) > kLdsMax) return launch_row<D>(p, n_cu, stream);
-  return launch_tile<D, kTileWaves, kTileRows>(p, stream);
+  // per workgroup).
+  if (rows <= n_cu) return launch_row<D>(p, n_cu, stream);
+  if (tile_lds_bytes<D, kTileWaves, kTileRows>(n_kv) <= kLdsMax) return launch_tile<D, kTileWaves, kTileRows>(p, stream);
+  switch (long_form<D>(n_kv, rows, n_cu)) {
+    case LongForm::kTile:
+      return launch_tile<D, 4, kTileRows>(p, stream);
+    case LongForm::kWave:
+      return launch_wave(p, stream);
+    default:
+      return launch_row<D>(p, n_cu, stream);
+  }
 }
 
 hipError_t launch_attn_exact(const ExactAttn& p, int n_cu, hipStream_t stream) {

@@ -132,14 +132,21 @@ def test_random_shapes_bit_for_bit(hip, stream, case):
     (1, 1, 128, 32127, 1),
     (1, 1, 128, 32128, 1),
     (1, 2, 128, 32767, 1),
-    (1, 1, 64, 0, 300),      # more rows than workgroups: tiles, from one key up
+    (1, 1, 64, 0, 300),      # more rows than workgroups and up to 300 keys: tiles
     (2, 7, 64, 63, 37),      # more rows than workgroups and few keys: staged, several a CU
     (2, 7, 64, 55, 73),      # 128 keys, and more rows than run at once: tiles
     (2, 7, 64, 56, 73),      # one key more: across a tile's edge
     (3, 5, 128, 3, 51),      # head_dim 128: 765 rows staged,
     (3, 5, 128, 3, 52),      # 780 in tiles, rows past the last
     (3, 5, 128, 60, 20),     # head_dim 128, 100 rows per KV head
-    (1, 8, 64, 4300, 40),    # more rows than workgroups, scores too long for tiles
+    (1, 8, 64, 4300, 40),    # more rows than workgroups, scores too long for tiles of 8 rows
+    (3, 6, 64, 4090, 30),    # more than two rounds of them: tiles of 4
+    (2, 9, 64, 4090, 70),    # more than one round of those: a wave per row
+    (2, 9, 64, 8150, 29),    # too long for tiles: rows
+    (3, 6, 128, 3100, 30),   # head_dim 128: tiles of 4,
+    (3, 6, 128, 6090, 29),   # then rows,
+    (3, 6, 128, 7600, 29),   # a wave per row where their buffers halve,
+    (3, 6, 128, 15000, 29),  # rows where fewer waves fit
 ])
 def test_row_and_tile_kernels_bit_for_bit(hip, stream, hkv, n_rep, d, n_past, n_tok):
     q, k, v = _inputs(77 + n_past, n_tok, n_past + n_tok, hkv * n_rep, hkv, d)
