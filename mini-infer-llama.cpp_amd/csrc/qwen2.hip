@@ -516,6 +516,15 @@ int load_model(const char* path, int32_t n_ctx, int32_t max_tokens, mi_hip_qwen2
   return MI_HIP_OK;
 }
 
+// A one-token step reads more than the caches hold, so each launch would find
+// its operands in HBM: idle CUs of one launch bring the next ones' into L2.
+// Of the cached K and V, which every XCD reads for itself, as much as about
+// fits in its 4 MB, from the first position on (us a token, without / these /
+// all of it: 24 layers of 2 KV heads of 64, reference order, 300 keys 1040 / 1013
+// / 1006, 6000 3357 / 3174 / 3182, 16000 7936 / 7788 / 7897; fused, 16000 1071 /
+// 1060 / 1328; 12 layers of 12 KV heads, 2400 keys 476 / 474 / 579).
+constexpr int64_t kWarmKvBytes = 5 << 20;
+
 // The activation of a projection: Q8_0_ACT blocks already in m->aq, or F32
 // columns x (x_ld floats apart) to quantise, after RMS_NORM * norm_w if set.
 struct Act {
@@ -580,10 +589,11 @@ int proj(const mi_hip_qwen2* m, const char* w, int64_t row_bytes, int64_t n, int
       p.rope = *rope;
       // the cached rows [0, pos) of this layer's K and V, position-major: a
       // step reads more weights than the caches hold, so attention would find
-      // them in HBM (24 layers, 300 keys: 1003 -> 965 us a token)
-      p.warm_bytes = (int64_t)rope->pos * m->kvd * 4;
-      p.warm[0] = rope->k_row - p.warm_bytes;
-      p.warm[1] = rope->v_row - p.warm_bytes;
+      // them in HBM
+      const int64_t past = (int64_t)rope->pos * m->kvd * 4;
+      p.warm_bytes = std::min(past, kWarmKvBytes / 2);
+      p.warm[0] = rope->k_row - past;
+      p.warm[1] = rope->v_row - past;
     } else {
       p.perm_hd = rope->hd;
       p.perm_rows = (int64_t)rope->n_q + rope->n_kv;
