@@ -163,11 +163,15 @@ __host__ __device__ inline int64_t q8_unperm_row(int64_t r, int32_t hd, int64_t 
 }
 // Whether launch_mul_mat_q8_0 takes the streaming form for p (the only form
 // with the activation prologue, and that for one column only).
+constexpr int kQ8RingMaxK = 960;  // its longest rows
 bool q8_ring_form(const Q8MulMat& p);
 // Whether launch_mul_mat_q8_0 can run p with its SwiGLU epilogue (the
 // streaming form, one column, no added term or RoPE, n a multiple of 64 and
 // at most one workgroup per 64 rows on the device).
 bool q8_swiglu_out_ok(const Q8MulMat& p, int n_cu);
+// Rows of the matrix per workgroup of the launch that launch_mul_mat_q8_0 makes
+// of p (one column), workgroup b the b-th so many; 0 if they are not dealt so.
+int q8_rows_per_workgroup(const Q8MulMat& p, int n_cu);
 hipError_t launch_quantize_q8_0_act(const Q8Quantize& p, hipStream_t stream);
 hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream);
 // mul_mat_cols.hip: several columns (k > 0, Q8_0_ACT blocks at p.a, no prologue or SwiGLU).

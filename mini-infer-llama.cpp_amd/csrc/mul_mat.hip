@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void mul_mat_q8_0_empty_kernel(const Q8MulMat 
 constexpr int kQ8RowBytesMax = 1024;
 constexpr int kQ8RingWaves = 8;
 constexpr int kQ8Slot = 8 * kQ8RowBytesMax;
-constexpr int kQ8MaxBlocks = 30;                   // k <= 960
+constexpr int kQ8MaxBlocks = kQ8RingMaxK / 32;
 constexpr int kQ8Cols = 2;
 constexpr int kQ8ActBytesMax = kQ8Cols * kQ8MaxBlocks * 36;
 constexpr int kQ8RingTake = kQ8RingWaves * 2 * kQ8Slot + kQ8ActBytesMax;  // the group counter
@@ -717,9 +717,20 @@ bool q8_ring_form(const Q8MulMat& p) {
   const bool cols_ok = p.m == 1 || (p.m == 2 && p.n >= kQ8TwoColsRows && !p.x && !p.perm_hd && !p.rope_on);
   // rows 4-byte aligned: every group's byte range ends on a whole dword (the
   // resource's range check is per dword)
-  return p.w_nb1 <= kQ8RowBytesMax && p.k <= 960 && cols_ok && (8 * p.w_nb1) % 16 == 0 &&
+  return p.w_nb1 <= kQ8RowBytesMax && p.k <= kQ8RingMaxK && cols_ok && (8 * p.w_nb1) % 16 == 0 &&
          p.w_nb1 % 4 == 0 &&
          reinterpret_cast<uintptr_t>(p.w) % 16 == 0 && act_ok && p.n * p.w_nb1 < (int64_t)1 << 40;
+}
+
+// The staged forms: 16-byte aligned groups of 8 rows that fit in LDS.
+static bool q8_staged_form(const Q8MulMat& p) {
+  return q8_stage_lds_bytes(p.w_nb1, p.k) <= kQ8StageLdsMax && reinterpret_cast<uintptr_t>(p.w) % 16 == 0 &&
+         (8 * p.w_nb1) % 16 == 0 && p.a_nb1 % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 4 == 0;
+}
+
+int q8_rows_per_workgroup(const Q8MulMat& p, int n_cu) {
+  if (q8_ring_form(p)) return p.n % 64 == 0 && p.n / 64 <= (n_cu > 0 ? n_cu : 256) ? 8 * kQ8RingWaves : 0;
+  return q8_staged_form(p) ? 8 : 0;
 }
 
 hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) {
@@ -771,8 +782,7 @@ hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) 
     return hipGetLastError();
   }
   if (p.m > 1) return launch_mul_mat_q8_0_cols(p, n_cu, stream);
-  if (q8_stage_lds_bytes(p.w_nb1, p.k) <= kQ8StageLdsMax && reinterpret_cast<uintptr_t>(p.w) % 16 == 0 &&
-      (8 * p.w_nb1) % 16 == 0 && p.a_nb1 % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 4 == 0) {
+  if (q8_staged_form(p)) {
     const dim3 grid((unsigned)((p.n + 7) / 8));
     if (q8_s1_ok(p)) {
       static const hipError_t attr1 = hipFuncSetAttribute((const void*)&mul_mat_q8_0_staged1_kernel,

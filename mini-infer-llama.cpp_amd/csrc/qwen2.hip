@@ -524,6 +524,12 @@ int load_model(const char* path, int32_t n_ctx, int32_t max_tokens, mi_hip_qwen2
 // / 1006, 6000 3357 / 3174 / 3182, 16000 7936 / 7788 / 7897; fused, 16000 1071 /
 // 1060 / 1328; 12 layers of 12 KV heads, 2400 keys 476 / 474 / 579).
 constexpr int64_t kWarmKvBytes = 5 << 20;
+// Of the next matrices (reference-order attention's launch), what fits in half
+// of the L2s together, once attention is long enough to hide it (us a token,
+// without / with: 24 layers of 896, 16 keys 872 / 903, 60 894 / 900, 150 928 /
+// 906, 300 1006 / 971, 2000 1655 / 1618).
+constexpr int64_t kWarmWeightBytes = 16 << 20;
+constexpr int kWarmWeightsFrom = 96;
 
 // The activation of a projection: Q8_0_ACT blocks already in m->aq, or F32
 // columns x (x_ld floats apart) to quantise, after RMS_NORM * norm_w if set.
@@ -627,10 +633,22 @@ int quantize_cols(const mi_hip_qwen2* m, const float* src, int64_t ne0, int64_t 
   return e == hipSuccess ? MI_HIP_OK : mi::rt_hip_fail(e, "qwen2 quantize launch");
 }
 
-// The rows of a matrix as the one-column streaming form deals them to its
-// workgroups (64 each while there are fewer of those than CUs).
-mi::WarmUp q8_warm_up(const char* w, int64_t row_bytes, int64_t rows) {
-  return {w, (int32_t)(64 * row_bytes), rows / 64 <= mi::rt_n_cu() ? (int32_t)(rows / 64) : 0};
+// A matrix of n rows as its one-column launch will deal them to its
+// workgroups, out of the `left` bytes that are still to be warmed up; nothing
+// where that is not known or it is more.
+mi::WarmUp q8_warm_up(const mi_hip_qwen2* m, const char* w, int64_t row_bytes, int64_t n, int64_t k, int64_t* left) {
+  mi::Q8MulMat p{};
+  p.w = w;
+  p.a = m->aq;
+  p.w_nb1 = row_bytes;
+  p.a_nb1 = k / 32 * 36;
+  p.k = k;
+  p.n = n;
+  p.m = 1;
+  const int rows = mi::q8_rows_per_workgroup(p, mi::rt_n_cu());
+  if (!rows || n * row_bytes > *left) return {};
+  *left -= n * row_bytes;
+  return {w, (int32_t)(rows * row_bytes), (int32_t)(n / rows)};
 }
 
 // Enqueues one forward pass on the model's stream, nothing waited for: the T
@@ -744,13 +762,15 @@ int enqueue_forward(mi_hip_qwen2* m, const int32_t* ids_dev, int T, int n_past, 
       ea.scale = scale;
       ea.aq = m->aq;
       ea.aq_ld = E / 32 * 36;
-      if (T == 1) {
-        // the CUs without a head bring the next matrices into L2 (together
-        // with one round of parameter loads per launch 1048 -> 1003 us a token)
-        ea.warm[0] = q8_warm_up(w.wo, m->row_e, E);
-        ea.warm[1] = q8_warm_up(w.wgu, m->row_e, 2 * (int64_t)F);
-        ea.warm[2] = {w.wdown, (int32_t)(8 * m->row_f), E / 8};
-        if (l + 1 < hp.n_layer) ea.warm[3] = q8_warm_up(m->layers[l + 1].wqkv, m->row_e, qkv_rows);
+      if (T == 1 && n_past >= kWarmWeightsFrom) {
+        // the CUs without a head bring the next matrices into L2
+        // (not where a row of E is too long for the streaming form: matrices that
+        // size pass through L2; 1536 wide, 2000 keys 843 us without, 852 with)
+        int64_t left = E <= mi::kQ8RingMaxK ? kWarmWeightBytes : 0;
+        ea.warm[0] = q8_warm_up(m, w.wo, m->row_e, E, E, &left);
+        ea.warm[1] = q8_warm_up(m, w.wgu, m->row_e, 2 * (int64_t)F, E, &left);
+        ea.warm[2] = q8_warm_up(m, w.wdown, m->row_f, E, F, &left);
+        if (l + 1 < hp.n_layer) ea.warm[3] = q8_warm_up(m, m->layers[l + 1].wqkv, m->row_e, qkv_rows, E, &left);
       }
       Q2_TRY(mi::launch_attn_exact(ea, mi::rt_n_cu(), st), "reference-order attention launch");
     } else if ((rc = mi_hip_attn_fwd(&aa))) {
