@@ -134,9 +134,9 @@ __global__ __launch_bounds__(256) void mul_mat_q8_0_empty_kernel(const Q8MulMat 
 }
 
 // The streaming form, for weight rows of at most 1 KB (k <= 960: every matrix
-// of a 896-wide model), 16-byte aligned groups of 8 rows and one column (or
-// two of a very tall matrix: q8_ring_form). One workgroup of 8 waves per CU; each wave walks row groups (8
-// rows) g = wave_id, wave_id + stride, ... through a ring of 2 LDS slots
+// of a 896-wide model), 16-byte aligned groups of 8 rows and one column (or two
+// or three of a very tall matrix: q8_ring_cols). One workgroup of 8 waves per
+// CU; each wave walks row groups (8 rows) of its range through a ring of 2 LDS slots
 // filled by buffer_load ... lds (16 bytes per lane, one resource per group
 // bounded at the tensor's end, so bytes past it arrive as zeros without a
 // request, and a group past the end refills through a zero-sized resource).
@@ -147,7 +147,7 @@ constexpr int kQ8RowBytesMax = 1024;
 constexpr int kQ8RingWaves = 8;
 constexpr int kQ8Slot = 8 * kQ8RowBytesMax;
 constexpr int kQ8MaxBlocks = kQ8RingMaxK / 32;
-constexpr int kQ8Cols = 2;
+constexpr int kQ8Cols = 3;
 constexpr int kQ8ActBytesMax = kQ8Cols * kQ8MaxBlocks * 36;
 constexpr int kQ8RingTake = kQ8RingWaves * 2 * kQ8Slot + kQ8ActBytesMax;  // the group counter
 constexpr int kQ8RingLds = kQ8RingTake + 16;
@@ -706,15 +706,26 @@ bool q8_swiglu_out_ok(const Q8MulMat& p, int n_cu) {
          p.n / 64 <= (n_cu > 0 ? n_cu : 256) && q8_ring_form(p);
 }
 
-// Two columns only of a matrix tall enough that its bytes are what takes the
-// time (151936 x 896: 40.1 us against the column tiles' 47; 4864 x 896: 8.8
-// against 6.9; three columns of the tallest take 45 and 47).
-constexpr int64_t kQ8TwoColsRows = 65536;
+// A matrix larger than the L2s together passes through them once.
+static bool q8_beyond_l2(const Q8MulMat& p, int64_t mb) { return p.n * p.w_nb1 > mb << 20; }
+
+// Two or three columns only of matrices whose bytes are what takes the time,
+// with long rows (this form's products take as long for a short row). us, this
+// form against the column tiles, 2 columns: 151936 x 896 37.4 / 44.2, 50000 x
+// 896 17.0 / 18.8, 36000 x 896 (33 MB) 13.7 / 14.7, 32768 x 896 11.9 both, 24000
+// 10.5 / 10.0, 4864 7.7 / 6.3 (16384 7.7 / 8.0: not worth a rule of its own),
+// 151936 x 704 36.5 / 40.6, x 640 36.4 / 35.4. 3 columns: 151936 x 896 42.8 /
+// 44.3, x 832 42.9 / 44.5, x 768 42.3 / 40.8, 120000 x 896 35.4 / 36.0, 100000
+// 31.3 / 31.6, 65536 22.7 / 21.2.
+static bool q8_ring_cols(const Q8MulMat& p) {
+  if (p.x || p.perm_hd || p.rope_on) return false;
+  return p.m == 2 ? p.k > 640 && q8_beyond_l2(p, 32) : p.m == 3 && p.k > 768 && q8_beyond_l2(p, 96);
+}
 
 bool q8_ring_form(const Q8MulMat& p) {
   const bool act_ok = p.x ? (p.x_ld >= p.k && reinterpret_cast<uintptr_t>(p.x) % 4 == 0)
                           : (p.a_nb1 % 4 == 0 && reinterpret_cast<uintptr_t>(p.a) % 4 == 0);
-  const bool cols_ok = p.m == 1 || (p.m == 2 && p.n >= kQ8TwoColsRows && !p.x && !p.perm_hd && !p.rope_on);
+  const bool cols_ok = p.m == 1 || q8_ring_cols(p);
   // rows 4-byte aligned: every group's byte range ends on a whole dword (the
   // resource's range check is per dword)
   return p.w_nb1 <= kQ8RowBytesMax && p.k <= kQ8RingMaxK && cols_ok && (8 * p.w_nb1) % 16 == 0 &&
@@ -746,19 +757,21 @@ hipError_t launch_mul_mat_q8_0(const Q8MulMat& p, int n_cu, hipStream_t stream) 
   if (p.x && !rows_form) return hipErrorInvalidValue;  // the prologue exists in the streaming form only
   if (rows_form) {
     const bool epi = p.rope_on || p.perm_hd;
-    // A matrix larger than the L2s together passes through them once: asked for
-    // nontemporally (151936 x 896, 145 MB: 29.0 -> 25.4 us; the 9.3 MB of a gate
-    // and up pair are in L2 by then, where the hint gains nothing).
-    const bool nt = p.n * p.w_nb1 > (int64_t)32 << 20;
-    const auto fn = p.m == 2 ? mul_mat_q8_0_ring_kernel<2, false, true>
-                    : epi    ? mul_mat_q8_0_ring_kernel<1, true, false>
-                    : nt     ? mul_mat_q8_0_ring_kernel<1, false, true>
-                             : mul_mat_q8_0_ring_kernel<1, false, false>;
+    // What passes through the L2s once is asked for nontemporally (151936 x 896,
+    // 145 MB: 29.0 -> 25.4 us, two columns of it 38.4 -> 37.3; the 9.3 MB of a
+    // gate and up pair are in L2 by then, where the hint gains nothing).
+    const bool nt = q8_beyond_l2(p, 32);
+    const auto fn = p.m == 2   ? mul_mat_q8_0_ring_kernel<2, false, true>
+                    : p.m == 3 ? mul_mat_q8_0_ring_kernel<3, false, true>
+                    : epi      ? mul_mat_q8_0_ring_kernel<1, true, false>
+                    : nt       ? mul_mat_q8_0_ring_kernel<1, false, true>
+                               : mul_mat_q8_0_ring_kernel<1, false, false>;
     static const hipError_t attr = [] {
-      const void* fns[4] = {(const void*)&mul_mat_q8_0_ring_kernel<1, false, false>,
+      const void* fns[5] = {(const void*)&mul_mat_q8_0_ring_kernel<1, false, false>,
                             (const void*)&mul_mat_q8_0_ring_kernel<1, false, true>,
                             (const void*)&mul_mat_q8_0_ring_kernel<1, true, false>,
-                            (const void*)&mul_mat_q8_0_ring_kernel<2, false, true>};
+                            (const void*)&mul_mat_q8_0_ring_kernel<2, false, true>,
+                            (const void*)&mul_mat_q8_0_ring_kernel<3, false, true>};
       hipError_t e = hipSuccess;
       for (const void* f : fns)
         if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kQ8RingLdsAll);

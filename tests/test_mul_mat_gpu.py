@@ -133,9 +133,13 @@ def test_q8_0_strided_operands(hip, stream, oracle, k, n, m):
     (224, 900, 128),   # 7 blocks: the last stage re-reads one; tiles of 32 columns x 16 rows
     (896, 33, 17),     # tiles of 16 x 16, one row and one column past
     (4832, 47, 3),     # 151 blocks: the last stage re-reads one, of 38
+    (704, 44857, 2),   # 32 MB: still tiles
+    (704, 44863, 2),   # more: the streaming form with 2 columns, 7 rows in the last group
+    (832, 113867, 3),  # 96 MB: tiles
+    (832, 113875, 3),  # the streaming form with 3 columns
 ])
 def test_q8_0_columns_bitwise(hip, stream, oracle, k, n, m):
-    # Every tile shape of the several-column products, at its edges, against
+    # Every form and tile shape of the several-column products, at its edges, against
     # the oracle; and with activations so small that scale products and sums
     # are denormal, against the one-column kernels (the oracle's host process
     # may flush denormals).
