@@ -394,24 +394,30 @@ static hipError_t launch_tile(Q8MulMat p, hipStream_t stream) {
   static const hipError_t attr =
       hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * S::kBuf);
   if (attr != hipSuccess) return attr;
-  const int64_t n_jt = (p.n + S::kN - 1) / S::kN, per_it = (n_jt + 7) / 8 * 8;
+  // one launch, unless rows or columns are too many for one grid
   const int64_t most = INT32_MAX / S::kT;  // workgroups of a launch
-  if (per_it > most) return hipErrorInvalidValue;
-  // (one launch, unless the columns are too many for one grid)
-  const int64_t step = most / per_it * S::kM, m = p.m;
-  for (int64_t c0 = 0; c0 < m; c0 += step) {
-    p.m = std::min(step, m - c0);
-    const int64_t n_it = (p.m + S::kM - 1) / S::kM;
-    hipLaunchKernelGGL(fn, dim3((unsigned)(per_it * n_it)), dim3(S::kT), 2 * S::kBuf, stream, p, (int)n_jt, (int)n_it);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    p.a += step * p.a_nb1;
-    p.dst += step * p.dst_nb1;
-    p.rope.pos += (int32_t)step;
-    p.rope.q_out += step * p.rope.q_ld;
-    p.rope.k_row += step * p.rope.c_s2;
-    p.rope.v_row += step * p.rope.c_s2;
-    if (p.add) p.add += step * p.add_nb1;
+  const int64_t n_step = most / 8 * 8 * S::kN, n = p.n, m = p.m;
+  if (n > n_step && (p.rope_on || p.perm_hd)) return hipErrorInvalidValue;  // (their rows are not dealt in parts)
+  const Q8MulMat whole = p;
+  for (int64_t r0 = 0; r0 < n; r0 += n_step) {
+    p.n = std::min(n_step, n - r0);
+    const int64_t n_jt = (p.n + S::kN - 1) / S::kN, per_it = (n_jt + 7) / 8 * 8;
+    const int64_t m_step = most / per_it * S::kM;
+    for (int64_t c0 = 0; c0 < m; c0 += m_step) {
+      p.m = std::min(m_step, m - c0);
+      p.w = whole.w + r0 * p.w_nb1;
+      p.a = whole.a + c0 * p.a_nb1;
+      p.dst = whole.dst + r0 * p.dst_nb0 + c0 * p.dst_nb1;
+      if (p.add) p.add = whole.add + r0 * p.add_nb0 + c0 * p.add_nb1;
+      p.rope.pos = whole.rope.pos + (int32_t)c0;
+      p.rope.q_out = whole.rope.q_out + c0 * p.rope.q_ld;
+      p.rope.k_row = whole.rope.k_row + c0 * p.rope.c_s2;
+      p.rope.v_row = whole.rope.v_row + c0 * p.rope.c_s2;
+      const int64_t n_it = (p.m + S::kM - 1) / S::kM;
+      hipLaunchKernelGGL(fn, dim3((unsigned)(per_it * n_it)), dim3(S::kT), 2 * S::kBuf, stream, p, (int)n_jt, (int)n_it);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
   }
   return hipSuccess;
 }

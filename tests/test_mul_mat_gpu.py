@@ -183,3 +183,25 @@ def test_q8_0_no_blocks_gives_zeros(hip, stream, n, m):
     got = out.cpu().numpy()
     assert not bits(got[:, :n]).any()  # +0.0
     assert np.isnan(got[:, n:]).all()
+
+
+def test_q8_0_columns_of_more_rows_than_a_grid(hip, stream, oracle):
+    # 3 columns of 2^28 + 4096 rows of one block: the column tiles of so many
+    # rows take two launches. The matrix is 4096 rows over and over.
+    import torch
+    k, n0, m, reps = 32, 4096, 3, 65537
+    rng = np.random.default_rng(28)
+    w = q8_weights(rng, n0, k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    _, act, q = quantize_on_device(hip, stream, x)
+    dw = dev(w).repeat(reps, 1)
+    n = n0 * reps
+    out = torch.full((m, n), float("nan"), device="cuda")
+    wt = make_tensor(dw.data_ptr(), [k, n], [34, 34], type_=mh.MI_TYPE_Q8_0)
+    d = make_tensor(out.data_ptr(), [n, m], [4, 4 * n], op=mh.MI_OP_MUL_MAT, src=[wt, q])
+    hip.check(hip.mi_hip_op_mul_mat(ctypes.byref(d), stream))
+    torch.cuda.synchronize()
+    want = oracle.mul_mat_q8_0(w, oracle.quantize_q8_0_act(x), k, n0, m)
+    assert np.array_equal(bits(out[:, :n0].cpu().numpy()), bits(want))
+    got = out.view(torch.int32).view(m, reps, n0)
+    assert bool((got == got[:, :1]).all())
