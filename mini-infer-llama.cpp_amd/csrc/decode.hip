@@ -615,7 +615,14 @@ void decode_kernel(const DecodeParams p) {
       wait_vmem<C::WAIT_K>();
     // S^T = K Q^T: lane l's A operand is row hq of the sub-tile, elements
     // 8 qg + 32 kk + i. One accumulator per product term (independent MFMA
-    // chains), summed in a fixed order.
+    // chains), summed in a fixed order; with an F16 cache two, each with half
+    // of the large products and one with the small ones first: a sum is
+    // rounded where it is half as large and half as often. Against one
+    // accumulator for each term, and against the vector form's float products
+    // (relative error to 64 bits in 1e-7, 40 seeds, queries N(0, 1), x 4, x 12):
+    // 28/4 heads of 128, 8147 keys 2.33, 5.19, 7.23 (2.59, 7.14, 9.62; vector
+    // 2.67, 6.17, 9.52); 14/2 of 64, 32700 keys 2.48, 5.50, 8.09 (2.60, 6.42,
+    // 9.76; 2.80, 6.22, 9.71). The time is the same.
     const lds_t* const krow = ring + SOFF + hq * C::RB;
     f32x4 s1 = {0.f, 0.f, 0.f, 0.f}, s2 = s1, s3 = s1;
     if constexpr (F16) {
@@ -624,8 +631,12 @@ void decode_kernel(const DecodeParams p) {
       for (int kk = 0; kk < KK; ++kk) kh[kk] = lds_load<f16x8>(krow + 16 * ((qg + 4 * kk) ^ swz<NSLOT>(hq)));
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) {
-        s1 = mfma_k32(kh[kk], qh[kk], s1);
         s2 = mfma_k32(kh[kk], ql[kk], s2);
+      }
+#pragma unroll
+      for (int kk = 0; kk < KK; kk += 2) {
+        s1 = mfma_k32(kh[kk + 1], qh[kk + 1], s1);
+        s2 = mfma_k32(kh[kk], qh[kk], s2);
       }
     } else {
       bf16x8 kh[KK], kl[KK];

@@ -304,8 +304,9 @@ DecodePlan plan_decode(mi::DecodeItem* it, int n_items, int n_head_kv, int n_rep
       // heads, 4 layers at 2000 (3.9) 13.1 against 14.5, at 1000 (1.96) 11.7
       // against 10.9; 14/2 heads, one layer at 1000-4096 (1) 8.6-9.0 against
       // 7.1-7.4, 28/4 heads at 512 (1) 10.9 against 8.5.
-      // Error against 64 bits between the lines (24 seeds, 28/4 heads): mean
-      // 2.62e-7 whole, 2.66e-7 split at 8147, 2.50e-7 and 2.56e-7 at 4 x 2000.
+      // Both hold the cache exactly and sum in float; the matrix form's Q and P
+      // are f16 pairs, and its error against 64 bits is the smaller one
+      // (process_mf in decode.hip has the figures).
       if (autom && f16 && q.long_waves) keep = false;
       if (keep) {
         q.mf = p.mf;  // sub-tiles and workgroups both double: long_waves stands

@@ -133,12 +133,13 @@ def test_decode_f16_cache_shapes(hip, stream, oracle, n_rep, hkv, d, n_kv, decod
 
 # The library's own choice for an F16 cache (MI_HIP_DECODE_AUTO, no fixture):
 # heads split on the vector units where the split launch's waves stream fewer
-# than 4 sub-tiles (one layer of the 0.5B shape at n_kv 512-8192, the 7B shape
+# than 3 sub-tiles (one layer of the 0.5B shape at n_kv 512-4096, the 7B shape
 # at 512), whole on the matrix cores otherwise (32768; the 7B shape at 4096
-# and 8192).
+# and 8192), also between 3 and 4 (32700; the 7B shape at 8147).
 @pytest.mark.parametrize("n_rep,hkv,d,n_kv", [(7, 2, 64, 512), (7, 2, 64, 1024), (7, 2, 64, 4096),
-                                              (7, 2, 64, 8192), (7, 2, 64, 32768), (7, 4, 128, 512),
-                                              (7, 4, 128, 4096), (7, 4, 128, 8192)])
+                                              (7, 2, 64, 8192), (7, 2, 64, 32700), (7, 2, 64, 32768),
+                                              (7, 4, 128, 512), (7, 4, 128, 4096), (7, 4, 128, 8147),
+                                              (7, 4, 128, 8192)])
 def test_decode_f16_cache_default_choice(hip, stream, oracle, n_rep, hkv, d, n_kv):
     print("f16 decode, default kernel choice", n_rep, hkv, d, n_kv, flush=True)
     q, k, v = cpu_attention.make_inputs(1900 + n_kv + d, d, n_rep * hkv, hkv, n_kv, 1)
@@ -146,6 +147,37 @@ def test_decode_f16_cache_default_choice(hip, stream, oracle, n_rep, hkv, d, n_k
     got = fused(hip, stream, q, k, v, n_kv - 1, scale, f16=True)
     assert_close(got, ref_out(oracle, q, k, v, n_kv - 1, scale, f16=True), TOL_F32, "widened")
     assert_close(got, ref_out(oracle, q, k, v, n_kv - 1, scale), TOL_F16, "unrounded")
+
+
+# An F16 cache's default form keeps the precision of float products: the
+# relative error against 64 bits, means over seeds, of the default choice where
+# it runs whole on the matrix cores and the split would stream 3 to 4 sub-tiles
+# a wave, and of the split's arithmetic (the vector units).
+@pytest.mark.parametrize("n_rep,hkv,d,n_kv", [(7, 4, 128, 8147), (7, 2, 64, 32700)])
+@pytest.mark.parametrize("q_scale", [1.0, 4.0])
+def test_decode_f16_cache_default_no_less_precise(hip, stream, n_rep, hkv, d, n_kv, q_scale):
+    import torch
+    scale = float(np.float32(1) / np.sqrt(np.float32(d)))
+    err = {mh.MI_HIP_DECODE_AUTO: [], mh.MI_HIP_DECODE_VALU: []}
+    for seed in range(12):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        q = torch.randn((1, n_rep * hkv, d), device="cuda", generator=g) * q_scale
+        k, v = (torch.randn((n_kv, hkv, d), device="cuda", generator=g).half() for _ in range(2))
+        s = torch.matmul(q.double().view(hkv, n_rep, d), k.double().permute(1, 2, 0).contiguous()) * scale
+        want = torch.matmul(torch.softmax(s, -1), v.double().permute(1, 0, 2).contiguous()).view(1, -1, d)
+        try:
+            for mode, e in err.items():
+                hip.check(hip.mi_hip_set_decode_mode(mode))
+                out = torch.full_like(q, float("nan"))
+                a = mh.attn_args(q, out, n_rep, n_kv - 1, scale, stream, k=k, v=v)
+                hip.check(hip.mi_hip_attn_fwd(ctypes.byref(a)))
+                torch.cuda.synchronize()
+                e.append(float((out.double() - want).norm() / want.norm()))
+        finally:
+            hip.check(hip.mi_hip_set_decode_mode(mh.MI_HIP_DECODE_AUTO))
+    auto, valu = (float(np.mean(e)) for e in err.values())
+    print(f"default {auto:.3e} vector units {valu:.3e}", flush=True)
+    assert auto <= valu
 
 
 @pytest.fixture(params=[mh.MI_HIP_DECODE_MATRIX, mh.MI_HIP_DECODE_VALU, mh.MI_HIP_DECODE_STREAM],
