@@ -394,8 +394,9 @@ void decode_kernel(const DecodeParams p) {
   }
   // MF: this lane's B operand of QK, Q[head hq][8 qg + 32 kk + i] (i < 8), as
   // hi/lo pairs; zero for head columns past G. With an F16 cache a head whose
-  // largest |q| exceeds 2^14 is scaled by a power of two into the f16 range
-  // (undone on its scores).
+  // largest |q| is above 2^14, or below 1 (the low halves would fall under the
+  // f16 range: 2^-25 of error that large keys multiply), is scaled by a power
+  // of two (undone on its scores).
   constexpr int KK = D / 32, NT = D / 16;
   typedef typename std::conditional<F16, f16x8, bf16x8>::type op8_t;
   typedef typename std::conditional<F16, half4_t, bf16x4>::type op4_t;
@@ -558,8 +559,9 @@ void decode_kernel(const DecodeParams p) {
         for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(qf[kk][i]));
       amax = fmaxf(amax, __shfl_xor(amax, 16));
       amax = fmaxf(amax, __shfl_xor(amax, 32));
-      if (amax > 16384.f) {  // 2^-e with 2^e >= amax / 2^14: exact scaling
-        const int e = ilogbf(amax) - 13;
+      // amax outside [1, 2^14]: an exact scaling by 2^-e brings it to [2^13, 2^14)
+      if ((amax > 0.f && amax < 1.f) || amax > 16384.f) {
+        const int e = max(ilogbf(amax) - 13, -100);
         const float f = ldexpf(1.f, -e);
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk)

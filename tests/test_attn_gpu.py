@@ -206,6 +206,27 @@ def test_decode_f16_cache_large_queries(hip, stream, oracle, decode_mode):
     assert_close(got, ref_out(oracle, q, k, v, n_kv - 1, scale, f16=True), TOL_F32, "widened")
 
 
+@pytest.mark.parametrize("n_kv", [300, 8147])
+def test_decode_f16_cache_small_queries(hip, stream, n_kv, decode_mode):
+    # Queries of 1e-4 against keys of 1e4: ordinary scores, from query elements
+    # whose low halves are below the f16 range unless the head is scaled. The
+    # bound is ten times what float products show at ordinary queries (2.7e-7).
+    hkv, n_rep, d = 4, 7, 128
+    q, k, v = cpu_attention.make_inputs(77, d, n_rep * hkv, hkv, n_kv, 1)
+    q = (q * np.float32(1e-4)).astype(np.float32)
+    q[0, 3] *= np.float32(1e-30)  # one head whose scores vanish
+    k16 = (k * np.float32(1e4)).astype(np.float16)
+    v16 = v.astype(np.float16)
+    scale = float(np.float32(1) / np.sqrt(np.float32(d)))
+    got = fused(hip, stream, q, k16, v16, n_kv - 1, scale, f16=True)
+    want = np.empty(q.shape)
+    for h in range(n_rep * hkv):
+        s = k16[:, h // n_rep].astype(np.float64) @ q[0, h].astype(np.float64) * scale
+        p = np.exp(s - s.max())
+        want[0, h] = p @ v16[:, h // n_rep].astype(np.float64) / p.sum()
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 2.7e-6
+
+
 @pytest.fixture()
 def tuning(hip):
     """Sets decode planner knobs for one test and restores the defaults."""
