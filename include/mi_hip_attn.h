@@ -185,7 +185,7 @@ int mi_hip_set_prefill_mode(int32_t mode);
  *   MI_HIP_DECODE_AUTO (the default): the vector units (MI_HIP_DECODE_VALU)
  *     for an F32 cache; for an F16 cache the matrix cores, except for short
  *     launches whose heads can be split between workgroups so that each
- *     wave streams fewer than 3 sub-tiles of 16 positions (the split is a
+ *     wave streams at most about 2 sub-tiles of 16 positions (the split is a
  *     vector-unit form, faster there).
  * The split bf16 pairs of the matrix form carry ~2^-16 relative error per
  * product into the scores, so with an F32 cache it stays within the 1e-4 bar

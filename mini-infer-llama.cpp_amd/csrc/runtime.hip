@@ -177,7 +177,7 @@ struct DecodePlan {
   int n_wg = 0;    // workgroups with work (records)
   int grid_x = 0;  // the widest item's workgroups (grid rows are items)
   bool dyn = false;     // dynamic sub-tile claims
-  bool long_waves = false;  // every wave streams 3 or more sub-tiles on average (streaming: stream_min)
+  bool long_waves = false;  // a wave streams more than 2 1/8 sub-tiles on average (streaming: stream_min)
   bool mf = false;      // matrix-core kernel
   bool stream = false;  // the streaming kernel (decode_stream.hip)
 };
@@ -255,7 +255,7 @@ void plan_items(DecodePlan& p, mi::DecodeItem* it, int n_items, int gpi, int wav
   }
   for (int i = 0; i < n_items; ++i) p.grid_x = std::max(p.grid_x, gpi * it[i].kpg);
   p.n_wg = (int)wg;
-  p.long_waves = sub >= 3 * wg * waves;
+  p.long_waves = 8 * sub > 17 * wg * waves;
 }
 
 // max_groups: the workspace's group capacity (a head split must fit in it).
@@ -295,15 +295,14 @@ DecodePlan plan_decode(mi::DecodeItem* it, int n_items, int n_head_kv, int n_rep
       bool keep = true;
       for (int i = 0; i < n_items; ++i) keep = keep && it[i].kpg >= kpg0[i];
       // An F16 cache takes the split (vector units) only where the split
-      // launch's waves stream fewer than 3 sub-tiles each on average; longer
-      // streams run faster whole on the matrix cores. F16, with the split's
-      // sub-tiles per wave (a row one tile short of a round number is as long as
-      // the round one: the line is not at 4): 28/4 heads, D 128, one layer at
-      // n_kv 8192 (4) 10.7 us against 14.5 split, at 8147 (3.98) 10.7 against
-      // 14.4; 14/2 heads, D 64, 4 layers at 8147 (3.98) 10.5 against 14.0; 28/4
-      // heads, 4 layers at 2000 (3.9) 13.1 against 14.5, at 1000 (1.96) 11.7
-      // against 10.9; 14/2 heads, one layer at 1000-4096 (1) 8.6-9.0 against
-      // 7.1-7.4, 28/4 heads at 512 (1) 10.9 against 8.5.
+      // launch's waves stream at most about 2 sub-tiles each on average; longer
+      // streams run faster whole on the matrix cores. F16, us split against
+      // whole, with the split's sub-tiles per wave: 14/2 heads, D 64, 12 layers
+      // at n_kv 600 (0.9) 7.7 / 8.9, 1000 (1.6) 8.9 / 9.3, 1300 (2) 10.0 / 9.3,
+      // 1600 (2.5) 10.6 / 9.3, 2000 (3.1) 12.6 / 9.6; 8 layers at 1700 (1.7) 9.0 /
+      // 9.6, 2100 (2.1) 9.9 / 9.5; 28/4 heads, D 128, 4 layers at 950 (1.9) 10.8 /
+      // 11.6, 1040 (2.03) 11.5 / 11.7, 1310 (2.6) 12.7 / 12.4, 2000 (3.9) 14.5 /
+      // 12.9; one layer at 8147 (3.98) 14.4 / 10.6.
       // Both hold the cache exactly and sum in float; the matrix form's Q and P
       // are f16 pairs, and its error against 64 bits is the smaller one
       // (process_mf in decode.hip has the figures).

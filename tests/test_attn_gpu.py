@@ -133,8 +133,8 @@ def test_decode_f16_cache_shapes(hip, stream, oracle, n_rep, hkv, d, n_kv, decod
 
 # The library's own choice for an F16 cache (MI_HIP_DECODE_AUTO, no fixture):
 # heads split on the vector units where the split launch's waves stream fewer
-# than 3 sub-tiles (one layer of the 0.5B shape at n_kv 512-4096, the 7B shape
-# at 512), whole on the matrix cores otherwise (32768; the 7B shape at 4096
+# than 2 1/8 sub-tiles (one layer of the 0.5B shape at n_kv 512-4096, the 7B
+# shape at 512), whole on the matrix cores otherwise (32768; the 7B shape at 4096
 # and 8192), also between 3 and 4 (32700; the 7B shape at 8147).
 @pytest.mark.parametrize("n_rep,hkv,d,n_kv", [(7, 2, 64, 512), (7, 2, 64, 1024), (7, 2, 64, 4096),
                                               (7, 2, 64, 8192), (7, 2, 64, 32700), (7, 2, 64, 32768),
