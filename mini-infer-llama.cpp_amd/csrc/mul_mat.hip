@@ -148,7 +148,7 @@ constexpr int kQ8RingWaves = 8;
 constexpr int kQ8Slot = 8 * kQ8RowBytesMax;
 constexpr int kQ8MaxBlocks = kQ8RingMaxK / 32;
 constexpr int kQ8Cols = 3;
-constexpr int kQ8ActBytesMax = kQ8Cols * kQ8MaxBlocks * 36;
+constexpr int kQ8ActBytesMax = (kQ8Cols * kQ8MaxBlocks * 36 + 15) & ~15;
 constexpr int kQ8RingTake = kQ8RingWaves * 2 * kQ8Slot + kQ8ActBytesMax;  // the group counter
 constexpr int kQ8RingLds = kQ8RingTake + 16;
 constexpr int kQ8XOff = kQ8RingLds;                // one F32 column's squares (M = 1), past the ring,
@@ -157,6 +157,8 @@ constexpr int kQ8SumWork = kQ8XOff + 4 * kQ8SqN;   // the 8-wave ordered sum's w
 constexpr int kQ8SwTab = kQ8SumWork + 64 + 8 * kWave * 4;  // SwiGLU epilogue: expf's table
 constexpr int kQ8SwVals = kQ8SwTab + 32 * 8;                 // and the workgroup's 32 values
 constexpr int kQ8RingLdsAll = kQ8SwVals + 32 * 4;
+// (misaligned, the sum's 16-byte reads cost a decode step 340 us)
+static_assert(kQ8XOff % 16 == 0 && kQ8SumWork % 16 == 0 && kQ8SwTab % 16 == 0, "16-byte aligned LDS regions");
 
 // A load of two floats that the compiler does not track, so that it never
 // makes the products wait for it (its register allocation otherwise sometimes
