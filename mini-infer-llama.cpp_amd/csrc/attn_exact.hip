@@ -602,12 +602,13 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
 }
 
 // ---------------------------------------------------------------------------
-// Many rows: the T n_rep rows (token, head) of one KV head, R consecutive ones
-// per wave, W waves per workgroup. Tiles of 64 keys come through two LDS
-// buffers, first all of K, then all of V, each request a tile ahead. Per tile
-// a wave forms its rows' scores with one key per lane (the queries are
-// uniform: scalar loads), later its rows' sums with one output element per
-// lane (two at D = 128); in between, lane r runs row r's ordered sum.
+// Many rows: the T n_rep rows (token, head) of one KV head, one per wave, W
+// waves per workgroup. Tiles of 64 keys come through two LDS buffers, first all
+// of K, then all of V, each request a tile ahead. Per tile a wave forms its
+// row's scores with one key per lane (the query is uniform: scalar loads),
+// later the row's sums with one output element per lane (two at D = 128); in
+// between, the ordered sum of the exponentials. (Two rows a wave, sharing its
+// reads: 128 tokens 10.1 us, with one 7.9, 384 tokens 23.8 and 20.1.)
 //
 // The vector units and LDS reads bound it: two vector instructions per product
 // (the order forbids the fused one), 4 D per (row, key) in all, and every
@@ -615,15 +616,15 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
 // heads, D 64, us; before: a workgroup with its own copy of K and V per row):
 // 128 tokens 11.2 -> 7.9, 384 tokens 123.8 -> 20.1.
 constexpr int kTileKeys = 64;
-// floats per row of scores: whole tiles, plus 4 so that the rows of a wave
-// start in different banks (and 16 readable past the last)
+// floats per row of scores: whole tiles, plus 4 so that the waves' rows start
+// in different banks (and 16 readable past the last)
 __host__ __device__ inline int tile_row_floats(int n) { return ((n + 63) & ~63) + 4; }
-template <int D, int W, int R>
+template <int D, int W>
 constexpr int tile_lds_bytes(int n) {
-  return 2 * kTileKeys * D * 4 + 256 + 4 * W * R * tile_row_floats(n) + 64;
+  return 2 * kTileKeys * D * 4 + 256 + 4 * W * tile_row_floats(n) + 64;
 }
 
-template <int D, int W, int R>
+template <int D, int W>
 __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAttn p, int n_tiles) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) char ex_lds[];
@@ -637,21 +638,14 @@ __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAt
   const int tile = n_tiles - 1 - blockIdx.x / n_hkv;  // the longest rows first
   const int np = tile_row_floats(p.n_past + p.n_tokens);
   lds_t* const tab = lds + 2 * kBuf;
-  lds_t* const sc = tab + 256 + 4 * np * R * wv;  // this wave's rows
+  lds_t* const sc = tab + 256 + 4 * np * wv;  // this wave's scores
   const char* const kbase = p.k + kvh * p.k_s1;
   const char* const vbase = p.v + kvh * p.v_s1;
-  // the wave's rows (past the last: the last again, not stored) and their keys
-  const int r0 = (tile * W + wv) * R;
-  int a[R];
-  const char* q[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const int r = min(r0 + i, n_rows - 1), j = r / p.n_rep, h = kvh * p.n_rep + (r - j * p.n_rep);
-    a[i] = p.n_past + j + 1;
-    q[i] = p.q + h * p.q_s1 + (int64_t)j * p.q_s2;
-  }
-  const int a_lo = a[0], a_hi = a[R - 1];  // a wave's rows have ascending key counts
-  const int a_wg = p.n_past + min((tile + 1) * W * R - 1, n_rows - 1) / p.n_rep + 1;
+  // the wave's row (past the last: the last again, not stored) and its keys
+  const int r = min(tile * W + wv, n_rows - 1), j = r / p.n_rep, h = kvh * p.n_rep + (r - j * p.n_rep);
+  const int a = p.n_past + j + 1;
+  const char* const q = p.q + h * p.q_s1 + (int64_t)j * p.q_s2;
+  const int a_wg = p.n_past + min((tile + 1) * W - 1, n_rows - 1) / p.n_rep + 1;
   const int nt = (a_wg + kTileKeys - 1) / kTileKeys;
   const uint64_t te = kExpfTab[lane & 31];
   if (tid < 32) lds_store<uint64_t>(tab + 8 * tid, te);
@@ -663,69 +657,49 @@ __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAt
       rows_to_lds<D, W, false>(b, vbase, p.v_s2, (s - nt) * kTileKeys, kTileKeys, a_wg - 1, wv, lane);
   };
   request(0);
-  float mx[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) mx[i] = -INFINITY;
+  float mx = -INFINITY;
   for (int s = 0; s < nt; ++s) {
     wait_vmem<0>();
     wg_barrier();  // tile s has landed, and everyone has left the other buffer
     request(s + 1);
     const int k0 = s * kTileKeys;
-    if (k0 >= a_hi) continue;
+    if (k0 >= a) continue;
     const lds_t* const rowp = lds + (s & 1) * kBuf + lane * (4 * D);
-    float acc[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) acc[i] = 0.0f;
+    float acc = 0.0f;
 #pragma unroll
     for (int u0 = 0; u0 < PPR; u0 += 4) {
       f32x4_t kv[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) kv[u] = lds_load<f32x4_t>(rowp + 16 * ((u0 + u) ^ swz<PPR>(lane)));
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-          // uniform address: a scalar load
-          const f32x4_t qv = *(const __attribute__((address_space(4))) f32x4_t*)(q[i] + 16 * (u0 + u));
-          acc[i] = acc[i] + kv[u].x * qv.x;
-          acc[i] = acc[i] + kv[u].y * qv.y;
-          acc[i] = acc[i] + kv[u].z * qv.z;
-          acc[i] = acc[i] + kv[u].w * qv.w;
-        }
+      for (int u = 0; u < 4; ++u) {
+        // uniform address: a scalar load
+        const f32x4_t qv = *(const __attribute__((address_space(4))) f32x4_t*)(q + 16 * (u0 + u));
+        acc = acc + kv[u].x * qv.x;
+        acc = acc + kv[u].y * qv.y;
+        acc = acc + kv[u].z * qv.z;
+        acc = acc + kv[u].w * qv.w;
+      }
     }
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const float v = acc[i] * p.scale;
-      lds_store<float>(sc + 4 * (i * np + k0 + lane), v);
-      mx[i] = k0 + lane < a[i] && v > mx[i] ? v : mx[i];
-    }
+    const float v = acc * p.scale;
+    lds_store<float>(sc + 4 * (k0 + lane), v);
+    mx = k0 + lane < a && v > mx ? v : mx;
   }
-  // exponentials, zeros past a row's keys (they leave its sum unchanged)
-  const int n_pad = (a_hi + 15) & ~15;
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    mx[i] = wave_max_dpp(mx[i]);  // (never NaN; the sign of a zero maximum changes no exponential)
-    for (int t = lane; t < n_pad; t += kWave) {
-      const float x = lds_load<float>(sc + 4 * (i * np + t)) - mx[i];
-      lds_store<float>(sc + 4 * (i * np + t),
-                       t < a[i] ? expf_ref(x, (const __attribute__((address_space(3))) uint64_t*)tab) : 0.0f);
-    }
+  // exponentials, zeros past the row's keys (they leave its sum unchanged)
+  const int n_pad = (a + 15) & ~15;
+  mx = wave_max_dpp(mx);  // (never NaN; the sign of a zero maximum changes no exponential)
+  for (int t = lane; t < n_pad; t += kWave) {
+    const float x = lds_load<float>(sc + 4 * t) - mx;
+    lds_store<float>(sc + 4 * t, t < a ? expf_ref(x, (const __attribute__((address_space(3))) uint64_t*)tab) : 0.0f);
   }
   wave_lds_fence();
-  const float sum = exact_sum(sc + 4 * np * min(lane, R - 1), n_pad, 0.0f);
-  const float inv_l = (float)(1.0 / (double)sum);  // the correctly rounded 1.0f / sum
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const float inv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv_l), i));
-    for (int t = lane; t < n_pad; t += kWave)
-      lds_store<float>(sc + 4 * (i * np + t), lds_load<float>(sc + 4 * (i * np + t)) * inv);
-  }
+  const float sum = exact_sum(sc, n_pad, 0.0f);
+  const float inv = (float)(1.0 / (double)sum);  // the correctly rounded 1.0f / sum
+  for (int t = lane; t < n_pad; t += kWave) lds_store<float>(sc + 4 * t, lds_load<float>(sc + 4 * t) * inv);
   wave_lds_fence();
-  float acc[R][ND];
+  float acc[ND];
 #pragma unroll
-  for (int i = 0; i < R; ++i)
-#pragma unroll
-    for (int d = 0; d < ND; ++d) acc[i][d] = 0.0f;
+  for (int d = 0; d < ND; ++d) acc[d] = 0.0f;
   for (int s = 0; s < nt; ++s) {
     wait_vmem<0>();
     wg_barrier();
@@ -733,44 +707,30 @@ __global__ __launch_bounds__(W* kWave) void attn_exact_tile_kernel(const ExactAt
     const int k0 = s * kTileKeys;
     const lds_t* const vb = lds + ((nt + s) & 1) * kBuf + 4 * lane;
     const lds_t* const pb = sc + 4 * k0;
-    // keys every row of the wave sees, 4 at a time, then the others one by one
-    const int n4 = max(min(a_lo - k0, kTileKeys), 0) >> 2, n1 = min(a_hi - k0, kTileKeys);
+    // the row's keys of the tile, 4 at a time, then the others one by one
+    const int n1 = min(a - k0, kTileKeys), n4 = max(n1, 0) >> 2;
 #pragma unroll 4
     for (int t4 = 0; t4 < n4; ++t4) {
       float v[4][ND];
-      f32x4_t pr[R];
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int d = 0; d < ND; ++d) v[t][d] = lds_load<float>(vb + (4 * t4 + t) * (4 * D) + 4 * kWave * d);
-#pragma unroll
-      for (int i = 0; i < R; ++i) pr[i] = lds_load<f32x4_t>(pb + 4 * (i * np + 4 * t4));
+      const f32x4_t pr = lds_load<f32x4_t>(pb + 16 * t4);
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int i = 0; i < R; ++i)
-#pragma unroll
-          for (int d = 0; d < ND; ++d) acc[i][d] = acc[i][d] + v[t][d] * pr[i][t];
+        for (int d = 0; d < ND; ++d) acc[d] = acc[d] + v[t][d] * pr[t];
     }
     for (int t = 4 * n4; t < n1; ++t) {
+      const float pt = lds_load<float>(pb + 4 * t);
 #pragma unroll
-      for (int i = 0; i < R; ++i)
-        if (k0 + t < a[i]) {
-          const float pt = lds_load<float>(pb + 4 * (i * np + t));
-#pragma unroll
-          for (int d = 0; d < ND; ++d)
-            acc[i][d] = acc[i][d] + lds_load<float>(vb + t * (4 * D) + 4 * kWave * d) * pt;
-        }
+      for (int d = 0; d < ND; ++d) acc[d] = acc[d] + lds_load<float>(vb + t * (4 * D) + 4 * kWave * d) * pt;
     }
   }
+  if (tile * W + wv < n_rows) {
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const int r = r0 + i;
-    if (r < n_rows) {
-      const int j = r / p.n_rep, h = kvh * p.n_rep + (r - j * p.n_rep);
-#pragma unroll
-      for (int d = 0; d < ND; ++d) store_out(p, j, h, kWave * d + lane, acc[i][d]);
-    }
+    for (int d = 0; d < ND; ++d) store_out(p, j, h, kWave * d + lane, acc[d]);
   }
 }
 
@@ -876,15 +836,14 @@ static hipError_t launch_row(const ExactAttn& p, int n_cu, hipStream_t stream) {
   return launch_row<D, 14 * 1024, D == 64 ? 48 : 16>(p, n_cu, stream);
 }
 
-template <int D, int W, int R>
+template <int D, int W>
 static hipError_t launch_tile(const ExactAttn& p, hipStream_t stream) {
-  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_tile_kernel<D, W, R>,
+  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_tile_kernel<D, W>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
   if (attr != hipSuccess) return attr;
-  const int rows = p.n_tokens * p.n_rep;
-  const int n_tiles = (rows + W * R - 1) / (W * R);
-  const unsigned lds = (unsigned)tile_lds_bytes<D, W, R>(p.n_past + p.n_tokens);
-  hipLaunchKernelGGL((attn_exact_tile_kernel<D, W, R>), dim3((unsigned)(n_tiles * (p.n_head / p.n_rep))),
+  const int n_tiles = (p.n_tokens * p.n_rep + W - 1) / W;
+  const unsigned lds = (unsigned)tile_lds_bytes<D, W>(p.n_past + p.n_tokens);
+  hipLaunchKernelGGL((attn_exact_tile_kernel<D, W>), dim3((unsigned)(n_tiles * (p.n_head / p.n_rep))),
                      dim3(W * kWave), lds, stream, p, n_tiles);
   return hipGetLastError();
 }
@@ -918,14 +877,10 @@ static LongForm long_form(int n_kv, int64_t rows, int n_cu) {
   const bool whole_buffers = row_lds_bytes(n_kv, 64 * 1024) <= kLdsMax;
   const double row = rounds(rows, n_cu) * (D == 64 ? (whole_buffers ? 14 : 15) : (whole_buffers ? 28.5 : 36));
   const double wave = whole * wave_round((double)per_cu) + (rest > 0 ? wave_round(rest) : 0);
-  const double tile = tile_lds_bytes<D, 4, 1>(n_kv) <= kLdsMax ? rounds(rows, 4 * n_cu) * (D == 64 ? 38 : 57) : row + 1;
+  const double tile = tile_lds_bytes<D, 4>(n_kv) <= kLdsMax ? rounds(rows, 4 * n_cu) * (D == 64 ? 38 : 57) : row + 1;
   if (row <= tile && row <= wave) return LongForm::kRow;
   return tile <= wave ? LongForm::kTile : LongForm::kWave;
 }
-
-// One row per wave: 128 tokens of 14 heads 7.9 us with 8 waves of 1 row, 10.1
-// with 8 of 2, 8.3 with 4 of 1; 384 tokens 20.1, 23.8 and 19.5.
-constexpr int kTileWaves = 8, kTileRows = 1;
 
 // Short rows: as many as run at once (LDS, and 5 or 3 waves' registers per
 // SIMD) and, where every row has a CU, up to the length at which the row kernel
@@ -950,10 +905,10 @@ static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
   // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.9 us, 41 a row
   // per workgroup).
   if (rows <= n_cu) return launch_row<D>(p, n_cu, stream);
-  if (tile_lds_bytes<D, kTileWaves, kTileRows>(n_kv) <= kLdsMax) return launch_tile<D, kTileWaves, kTileRows>(p, stream);
+  if (tile_lds_bytes<D, 8>(n_kv) <= kLdsMax) return launch_tile<D, 8>(p, stream);
   switch (long_form<D>(n_kv, rows, n_cu)) {
     case LongForm::kTile:
-      return launch_tile<D, 4, kTileRows>(p, stream);
+      return launch_tile<D, 4>(p, stream);
     case LongForm::kWave:
       return launch_wave(p, stream);
     default:
