@@ -13,13 +13,16 @@
 //   acts     x [n_embd, T] (the residual stream), qkv [n_embd + 2 kv, T],
 //            attention output [head_dim, n_head, T], gate/up pairs [2 n_ff, T],
 //            Q8_0 activation blocks for the widest input, logits [n_vocab, T].
-// Per layer: RMSNorm*w -> Q8_0 blocks (one kernel), QKV + bias (matrix
-// epilogue), RoPE + K/V append (one kernel), attention (decode or prefill
-// kernel), Q8_0 blocks of its output, O projection + residual (epilogue, in
-// place), RMSNorm*w -> blocks, gate/up with SiLU(gate)*up -> blocks (the
-// matrix kernel's epilogue for one column, a kernel of its own for several),
-// down projection + residual. Then the final norm of the returned columns,
-// the lm_head and an argmax on the device.
+// Per layer: RMSNorm*w -> Q8_0 blocks (the QKV product's prologue for one
+// column, a kernel of its own for several), QKV + bias with RoPE and the K/V
+// append as its epilogue (a kernel of its own for one column of a model wider
+// than the streaming form), attention, whose output the reference-order kernels
+// write as Q8_0 blocks (the fused ones as floats, quantised like the norms'
+// outputs), O projection + residual (epilogue, in place), RMSNorm*w -> blocks,
+// gate/up with SiLU(gate)*up -> blocks (the matrix kernel's epilogue for one
+// column, a kernel of its own for several), down projection + residual. Then
+// the final norm of the returned columns, the lm_head and an argmax on the
+// device.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -540,9 +543,9 @@ struct Act {
 
 int quantize_cols(const mi_hip_qwen2* m, const float* src, int64_t ne0, int64_t cols, char* dst);
 
-// dst[:, j] (+)= W . act[:, j] for j < m_cols. Decode-sized calls take the
-// streaming matrix kernel with the norm / quantisation as its prologue (one
-// launch); the others run the norm or quantize kernel into m->aq first.
+// dst[:, j] (+)= W . act[:, j] for j < m_cols. One column takes the streaming
+// matrix kernel with the norm / quantisation as its prologue (one launch) where
+// its rows fit; otherwise the norm or quantize kernel fills m->aq first.
 // With swiglu_out (rows in gate/up pairs), one column is written as the
 // Q8_0_ACT blocks of SiLU(gate) * up at swiglu_out when the matrix kernel's
 // epilogue takes the shape (*swiglued says whether it did; otherwise dst holds
