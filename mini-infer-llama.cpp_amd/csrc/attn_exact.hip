@@ -20,6 +20,7 @@
 // per wave on its own (attn_exact_wave_kernel).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "attn_common.h"
 #include "kernels.h"
@@ -128,11 +129,11 @@ __device__ __forceinline__ float exact_column(const lds_t* p, int n, float acc) 
 
 // Output element o (its lane's, in aligned groups of 32 lanes) of row (j, h).
 __device__ __forceinline__ void store_out(const ExactAttn& p, int j, int h, int o, float v) {
-  if (p.aq) {
+  if (p.blocks) {
     float d;
     const int q = q8_lane_quant(v, d);
     const int e = h * p.head_dim + o;
-    char* const blk = p.aq + (int64_t)j * p.aq_ld + 36 * (e / 32);
+    char* const blk = p.out + (int64_t)j * p.o_s2 + 36 * (e / 32);
     if ((e & 31) == 0) gstore<float>(blk, d);
     gstore<signed char>(blk + 4 + (e & 31), (signed char)q);
   } else {
@@ -177,7 +178,7 @@ __device__ __forceinline__ void rows_to_lds(lds_t* dst, const char* base, int64_
 // A workgroup past the rows: its share of what the next launches read, pieces
 // of its own XCD (the same workgroup number modulo 8).
 template <int T>
-__device__ __forceinline__ void warm_up(const ExactAttn& p) {
+__device__ __forceinline__ void warm_up(const ExactAttnWarm& p) {
   const int n_rows = p.n_tokens * p.n_head;
   const int xcd = blockIdx.x % 8, first = (n_rows + 7 - xcd) / 8, per_xcd = ((int)gridDim.x + 7 - xcd) / 8 - first;
   for (int w = 0, c = blockIdx.x / 8 - first; w < kMaxWarmUps; ++w) {
@@ -280,8 +281,8 @@ __device__ __forceinline__ float exact_dot(const lds_t* v, const lds_t* p, int n
   return acc;
 }
 
-template <int D>
-__global__ __launch_bounds__(kStagedThreads) void attn_exact_staged_kernel(const ExactAttn p) {
+template <int D, typename P>
+__global__ __launch_bounds__(kStagedThreads) void attn_exact_staged_kernel(const P p) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) char ex_lds[];
   lds_t* const lds = (lds_t*)ex_lds;
@@ -292,11 +293,12 @@ __global__ __launch_bounds__(kStagedThreads) void attn_exact_staged_kernel(const
   // every parameter in one round of scalar loads, not one where each is first used
   asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.q_s1), "s"(p.q_s2), "s"(p.k_s1), "s"(p.k_s2), "s"(p.v_s1),
                "s"(p.v_s2), "s"(p.n_head), "s"(p.n_rep), "s"(p.n_past), "s"(p.n_tokens), "s"(p.scale), "s"(p.out),
-               "s"(p.o_s1), "s"(p.o_s2), "s"(p.aq), "s"(p.aq_ld));
-  if ((int)blockIdx.x >= p.n_tokens * p.n_head) {
-    warm_up<kStagedThreads>(p);
-    return;
-  }
+               "s"(p.o_s1), "s"(p.o_s2), "s"(p.blocks));
+  if constexpr (std::is_same<P, ExactAttnWarm>::value)
+    if ((int)blockIdx.x >= p.n_tokens * p.n_head) {
+      warm_up<kStagedThreads>(p);
+      return;
+    }
   const int h = blockIdx.x % p.n_head;
   const int j = p.n_tokens - 1 - blockIdx.x / p.n_head;  // the longest rows first
   const int kvh = h / p.n_rep;
@@ -378,12 +380,12 @@ __global__ __launch_bounds__(kStagedThreads) void attn_exact_staged_kernel(const
 // (two at D = 128): four other waves form the products P_t V[t] into LDS, a
 // chunk ahead.
 //
-// Measured (14 / 2 heads, D 64, us per launch; before: one kernel with the
-// whole row in LDS up to 512 keys and one of a wave per row beyond): n_kv 129
-// 7.3 -> 6.7, 301 10.2 -> 8.0, 1501 75.4 -> 24.5. There the output chains take
-// 10.5 (7 ns a key, 4.2 of them the addition itself), the scores 6.7
-// (LDS-direct requests bring about 55 GB/s into a CU, and a row has one CU),
-// the exponentials and their sum 2.7.
+// Measured (14 / 2 heads, D 64, us per launch; before: the staged kernel up to
+// 512 keys, a wave of its own per row beyond): n_kv 301 9.6 -> 8.6, 1001 38.5 ->
+// 17.4, 1501 75.4 -> 24.5, 8001 391 -> 122. At 1501 the output chains take 10.5
+// (7 ns a key, 4.2 of them the addition itself), the scores 6.7 (LDS-direct
+// requests bring about 55 GB/s into a CU, and a row has one CU), the
+// exponentials and their sum 2.7.
 constexpr int kRowThreads = 512;
 constexpr int kRowWaves = kRowThreads / kWave;
 constexpr int kRowLoaders = 4;          // waves that form the products
@@ -398,8 +400,8 @@ static_assert(4 * (kExactMaxKeys + 16) + kRowWork + 2 * 14 * 1024 <= kLdsMax, "t
 
 // BUF: bytes of a buffer of K rows (two, whole requests of every wave), later
 // of CK rows of products.
-template <int D, int BUF, int CK>
-__global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const ExactAttn p) {
+template <int D, int BUF, int CK, typename P>
+__global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const P p) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) char ex_lds[];
   lds_t* const lds = (lds_t*)ex_lds;
@@ -414,10 +416,11 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
   // every parameter in one round of scalar loads, not one where each is first used
   asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.q_s1), "s"(p.q_s2), "s"(p.k_s1), "s"(p.k_s2), "s"(p.v_s1),
                "s"(p.v_s2), "s"(p.n_head), "s"(p.n_rep), "s"(p.n_past), "s"(p.n_tokens), "s"(p.scale));
-  if ((int)blockIdx.x >= p.n_tokens * p.n_head) {
-    warm_up<kRowThreads>(p);
-    return;
-  }
+  if constexpr (std::is_same<P, ExactAttnWarm>::value)
+    if ((int)blockIdx.x >= p.n_tokens * p.n_head) {
+      warm_up<kRowThreads>(p);
+      return;
+    }
   const int h = blockIdx.x % p.n_head;
   const int j = p.n_tokens - 1 - blockIdx.x / p.n_head;  // the longest rows first
   const int kvh = h / p.n_rep;
@@ -608,13 +611,13 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const Exact
 // row's scores with one key per lane (the query is uniform: scalar loads),
 // later the row's sums with one output element per lane (two at D = 128); in
 // between, the ordered sum of the exponentials. (Two rows a wave, sharing its
-// reads: 128 tokens 10.1 us, with one 7.9, 384 tokens 23.8 and 20.1.)
+// reads: 128 tokens 10.1 us, with one 7.4, 384 tokens 23.8 and 19.7.)
 //
 // The vector units and LDS reads bound it: two vector instructions per product
 // (the order forbids the fused one), 4 D per (row, key) in all, and every
 // operand of them read from LDS or through scalar loads. Measured (14 / 2
 // heads, D 64, us; before: a workgroup with its own copy of K and V per row):
-// 128 tokens 11.2 -> 7.9, 384 tokens 123.8 -> 20.1.
+// 128 tokens 10.9 -> 7.4, 384 tokens 123.8 -> 19.7.
 constexpr int kTileKeys = 64;
 // floats per row of scores: whole tiles, plus 4 so that the waves' rows start
 // in different banks (and 16 readable past the last)
@@ -795,35 +798,38 @@ __global__ __launch_bounds__(kWave) void attn_exact_wave_kernel(const ExactAttn 
 
 // Workgroups past the rows: what is to be warmed up gets the idle CUs, two
 // pieces each.
-static int side_workgroups(const ExactAttn& p, int n_cu) {
+static int side_workgroups(const ExactAttn&, int) { return 0; }
+static int side_workgroups(const ExactAttnWarm& p, int n_cu) {
   int64_t pieces = 0;
   for (const WarmUp& w : p.warm) pieces += w.n;
   return (int)std::min<int64_t>(std::max(n_cu - p.n_tokens * p.n_head, 0) & ~7, (pieces + 15) / 16 * 8);
 }
 
-template <int D>
-static hipError_t launch_staged(const ExactAttn& p, int n_cu, hipStream_t stream) {
-  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_staged_kernel<D>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
+template <int D, typename P>
+static hipError_t launch_staged(const P& p, int n_cu, hipStream_t stream) {
+  const auto fn = &attn_exact_staged_kernel<D, P>;
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
   if (attr != hipSuccess) return attr;
   const int rows = p.n_tokens * p.n_head;
-  hipLaunchKernelGGL(attn_exact_staged_kernel<D>, dim3((unsigned)(rows + side_workgroups(p, n_cu))),
-                     dim3(kStagedThreads), (unsigned)staged_lds_bytes(p.n_past + p.n_tokens, D), stream, p);
+  hipLaunchKernelGGL(fn, dim3((unsigned)(rows + side_workgroups(p, n_cu))), dim3(kStagedThreads),
+                     (unsigned)staged_lds_bytes(p.n_past + p.n_tokens, D), stream, p);
   return hipGetLastError();
 }
 
-template <int D, int BUF, int CK>
-static hipError_t launch_row(const ExactAttn& p, int n_cu, hipStream_t stream) {
-  static const hipError_t attr = hipFuncSetAttribute((const void*)&attn_exact_row_kernel<D, BUF, CK>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
+template <int D, int BUF, int CK, typename P>
+static hipError_t launch_row(const P& p, int n_cu, hipStream_t stream) {
+  const auto fn = &attn_exact_row_kernel<D, BUF, CK, P>;
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax);
   if (attr != hipSuccess) return attr;
   const int rows = p.n_tokens * p.n_head;
-  hipLaunchKernelGGL((attn_exact_row_kernel<D, BUF, CK>), dim3((unsigned)(rows + side_workgroups(p, n_cu))), dim3(kRowThreads),
+  hipLaunchKernelGGL(fn, dim3((unsigned)(rows + side_workgroups(p, n_cu))), dim3(kRowThreads),
                      (unsigned)row_lds_bytes(p.n_past + p.n_tokens, BUF), stream, p);
   return hipGetLastError();
 }
-template <int D>
-static hipError_t launch_row(const ExactAttn& p, int n_cu, hipStream_t stream) {
+template <int D, typename P>
+static hipError_t launch_row(const P& p, int n_cu, hipStream_t stream) {
   // the largest buffers that fit beside the probabilities; short rows start
   // their chains after half as many products
   const int n_kv = p.n_past + p.n_tokens;
@@ -902,7 +908,7 @@ static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
   const int64_t rows = (int64_t)p.n_tokens * p.n_head;
   if (staged_form<D>(n_kv, rows, n_cu)) return launch_staged<D>(p, n_cu, stream);
   // Rows that get a CU each take a workgroup each (14 rows of 1501 keys: 24.5
-  // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.9 us, 41 a row
+  // us, 57 in tiles); more share tiles (128 tokens x 14 heads: 7.4 us, 41 a row
   // per workgroup).
   if (rows <= n_cu) return launch_row<D>(p, n_cu, stream);
   if (tile_lds_bytes<D, 8>(n_kv) <= kLdsMax) return launch_tile<D, 8>(p, stream);
@@ -916,7 +922,19 @@ static hipError_t launch(const ExactAttn& p, int n_cu, hipStream_t stream) {
   }
 }
 
+template <int D>
+static hipError_t launch(const ExactAttnWarm& p, int n_cu, hipStream_t stream) {
+  const int64_t rows = (int64_t)p.n_tokens * p.n_head;
+  if (rows > n_cu) return launch<D>(static_cast<const ExactAttn&>(p), n_cu, stream);  // (no CU is idle)
+  return staged_form<D>(p.n_past + p.n_tokens, rows, n_cu) ? launch_staged<D>(p, n_cu, stream)
+                                                          : launch_row<D>(p, n_cu, stream);
+}
+
 hipError_t launch_attn_exact(const ExactAttn& p, int n_cu, hipStream_t stream) {
+  n_cu = n_cu > 0 ? n_cu : 256;
+  return p.head_dim == 64 ? launch<64>(p, n_cu, stream) : launch<128>(p, n_cu, stream);
+}
+hipError_t launch_attn_exact_warm(const ExactAttnWarm& p, int n_cu, hipStream_t stream) {
   n_cu = n_cu > 0 ? n_cu : 256;
   return p.head_dim == 64 ? launch<64>(p, n_cu, stream) : launch<128>(p, n_cu, stream);
 }

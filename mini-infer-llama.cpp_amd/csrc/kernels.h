@@ -204,16 +204,21 @@ struct ExactAttn {
   int64_t q_s1, q_s2, k_s1, k_s2, v_s1, v_s2, o_s1, o_s2;
   int32_t n_head, n_rep, n_past, n_tokens, head_dim;
   float scale;
-  // Optional: the output as Q8_0_ACT blocks (element h * head_dim + o of token j
-  // in block (h * head_dim + o) / 32 of the column at aq + j * aq_ld) instead of
-  // F32 at out -- the engine's QUANTIZE node before the output projection fused.
-  char* aq = nullptr;
-  int64_t aq_ld = 0;
-  // Optional (one-workgroup-per-row launches only): brought into L2 by the CUs
-  // that the rows leave idle.
-  WarmUp warm[kMaxWarmUps] = {};
+  // Nonzero: the output as Q8_0_ACT blocks (element h * head_dim + o of token j
+  // in block (h * head_dim + o) / 32 of the column at out + j * o_s2) instead of
+  // F32 -- the engine's QUANTIZE node before the output projection fused.
+  int32_t blocks;
+};
+// Launches of 128 bytes of arguments are enqueued 0.15 us sooner than of 200:
+// what only a decode step has is a type of its own.
+static_assert(sizeof(ExactAttn) <= 128, "two lines of kernel arguments");
+// A launch of at most one row per CU, with what the CUs that the rows leave
+// idle bring into L2.
+struct ExactAttnWarm : ExactAttn {
+  WarmUp warm[kMaxWarmUps];
 };
 hipError_t launch_attn_exact(const ExactAttn& p, int n_cu, hipStream_t stream);
+hipError_t launch_attn_exact_warm(const ExactAttnWarm& p, int n_cu, hipStream_t stream);
 
 // Host helpers of the library's entry points (runtime.hip), for the other
 // host files: the thread's last-error message, the accounted device

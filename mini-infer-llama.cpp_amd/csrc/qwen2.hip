@@ -744,38 +744,40 @@ int enqueue_forward(mi_hip_qwen2* m, const int32_t* ids_dev, int T, int n_past, 
       size_t knb[4], vnb[4];
       if ((rc = mi_hip_kv_view(m->kv, l, 0, &kd, ne, knb)) || (rc = mi_hip_kv_view(m->kv, l, 1, &vd, ne, vnb)))
         return rc;
-      mi::ExactAttn ea{};
+      mi::ExactAttnWarm ea{};
       ea.q = reinterpret_cast<const char*>(m->qkv);
       ea.k = static_cast<const char*>(kd);
       ea.v = static_cast<const char*>(vd);
-      ea.out = reinterpret_cast<char*>(m->ao);
+      ea.out = m->aq;
       ea.q_s1 = (int64_t)nb[1];
       ea.q_s2 = (int64_t)nb[2];
       ea.k_s1 = (int64_t)knb[1];
       ea.k_s2 = (int64_t)knb[2];
       ea.v_s1 = (int64_t)vnb[1];
       ea.v_s2 = (int64_t)vnb[2];
-      ea.o_s1 = 4 * (int64_t)hd;
-      ea.o_s2 = 4 * (int64_t)E;
+      ea.o_s2 = E / 32 * 36;
+      ea.blocks = 1;
       ea.n_head = H;
       ea.n_rep = H / hp.n_head_kv;
       ea.n_past = n_past;
       ea.n_tokens = T;
       ea.head_dim = hd;
       ea.scale = scale;
-      ea.aq = m->aq;
-      ea.aq_ld = E / 32 * 36;
-      if (T == 1 && n_past >= kWarmWeightsFrom) {
-        // the CUs without a head bring the next matrices into L2
-        // (not where a row of E is too long for the streaming form: matrices that
-        // size pass through L2; 1536 wide, 2000 keys 843 us without, 852 with)
-        int64_t left = E <= mi::kQ8RingMaxK ? kWarmWeightBytes : 0;
+      hipError_t e;
+      if (T == 1 && n_past >= kWarmWeightsFrom && E <= mi::kQ8RingMaxK) {
+        // the CUs without a head bring the next matrices into L2 (not where a
+        // row of E is too long for the streaming form: matrices that size pass
+        // through L2; 1536 wide, 2000 keys 843 us without, 852 with)
+        int64_t left = kWarmWeightBytes;
         ea.warm[0] = q8_warm_up(m, w.wo, m->row_e, E, E, &left);
         ea.warm[1] = q8_warm_up(m, w.wgu, m->row_e, 2 * (int64_t)F, E, &left);
         ea.warm[2] = q8_warm_up(m, w.wdown, m->row_f, E, F, &left);
         if (l + 1 < hp.n_layer) ea.warm[3] = q8_warm_up(m, m->layers[l + 1].wqkv, m->row_e, qkv_rows, E, &left);
+        e = mi::launch_attn_exact_warm(ea, mi::rt_n_cu(), st);
+      } else {
+        e = mi::launch_attn_exact(ea, mi::rt_n_cu(), st);
       }
-      Q2_TRY(mi::launch_attn_exact(ea, mi::rt_n_cu(), st), "reference-order attention launch");
+      Q2_TRY(e, "reference-order attention launch");
     } else if ((rc = mi_hip_attn_fwd(&aa))) {
       return rc;
     }
