@@ -15,13 +15,14 @@
 // multiply-adds is the int8 -> f16 conversion of the operands, once per
 // workgroup on their way into LDS.
 //
-// Measured (MI355X, us; before: one wave per 8 rows with integer dots, weight
-// rows in LDS, 8 columns at a time): 4864 x 896 with 512 columns 534 -> 41,
-// 9728 x 896 with 128 164 -> 21, 896 x 4864 with 128 543 -> 17, with 37 160 ->
-// 14, with 8 36 -> 14; 896 x 896 with 128 129 -> 6.4, with 8 (the streaming
-// form) 15 -> 6.3. 512 columns take 14 us of multiply-adds at one per 4
-// cycles and SIMD; issue slots (conversions, products, LDS) fill the rest: a
-// lone wave issues an instruction every 5 cycles or so.
+// Measured (MI355X, us, the product alone in launches back to back; before: one
+// wave per 8 rows with integer dots, weight rows in LDS, 8 columns at a time):
+// 4864 x 896 with 512 columns 532 -> 35, 9728 x 896 with 128 163 -> 19.5, 896 x
+// 4864 with 128 542 -> 15.6, with 37 161 -> 13.2, with 8 36 -> 13.1; 896 x 896
+// with 128 129 -> 5.8, with 8 (the streaming form) 15.1 -> 5.1. 512 columns take
+// 14 us of multiply-adds at one per 4 cycles and SIMD; issue slots (conversions,
+// products, LDS) fill the rest: a lone wave issues an instruction every 5 cycles
+// or so.
 #include <algorithm>
 #include <type_traits>
 
@@ -427,7 +428,7 @@ static hipError_t launch_tile(Q8MulMat p, hipStream_t stream) {
 // stages (896 x 4864 with 37 columns: 14.4 us in 168 tiles of 16 x 16, 16.1 in
 // 112 of 32 x 16, 25.7 in 56 of 32 x 32; with 128: 17.2 in 224 of 32 x 16, 20.7
 // in 448 of 16 x 16). At most 16 columns that do fill it take 16-column tiles
-// (151936 x 896 with 8: 47 us, 66 in tiles of 32).
+// (151936 x 896 with 8: 45 us, 66 in tiles of 32).
 hipError_t launch_mul_mat_q8_0_cols(const Q8MulMat& p, int n_cu, hipStream_t stream) {
   const int64_t cu = n_cu > 0 ? n_cu : 256;
   const int64_t j16 = (p.n + 15) / 16, i16 = (p.m + 15) / 16, i32 = (p.m + 31) / 32;
