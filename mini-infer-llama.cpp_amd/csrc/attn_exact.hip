@@ -489,7 +489,8 @@ __global__ __launch_bounds__(kRowThreads) void attn_exact_row_kernel(const P p) 
     }
     wait_vmem<kTouch>();  // the K rows
     wg_barrier();
-    if (tid < a) score(tid, buf + tid * (4 * D), tid);  // (the buffers are adjacent)
+    // (the buffers are adjacent; a row's slots are swizzled by its place in its own)
+    if (tid < a) score(tid, buf + tid * (4 * D), tid < KB ? tid : tid - KB);
 #pragma unroll
     for (int u = 0; u < kTouch; ++u) asm volatile("" ::"v"(vt[u]));
   } else {

@@ -152,3 +152,28 @@ def test_row_and_tile_kernels_bit_for_bit(hip, stream, hkv, n_rep, d, n_past, n_
     q, k, v = _inputs(77 + n_past, n_tok, n_past + n_tok, hkv * n_rep, hkv, d)
     _check(hip, stream, q, k, v, n_past, float(np.float32(d ** -0.5)),
            f"{hkv} x {n_rep} heads of {d}, {n_tok} rows after {n_past}")
+
+
+@pytest.mark.parametrize("d,n_tok", [
+    (64, 4000), (64, 7000), (128, 5000),   # tiles of 8 rows, of 4, of 4
+    (64, 4200), (128, 7000),               # a wave per row
+    (64, 20700), (64, 32300), (128, 20700), (128, 32300),  # rows, with K buffers of 16 and 14 KB
+])
+def test_short_rows_of_a_long_launch_bit_for_bit(hip, stream, d, n_tok):
+    # The kernel and its K buffers are those of a launch's longest row; its
+    # short rows come through the same ones. Rows of one key up to past both
+    # buffers, against one-row launches of their own (the oracle checks those
+    # above).
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n_tok + d)
+    q, k, v = (torch.randn((n_tok, 1, d), device="cuda", generator=g) for _ in range(3))
+    scale = float(np.float32(d ** -0.5))
+    out = torch.full_like(q, float("nan"))
+    a = mh.attn_args(q, out, 1, 0, scale, stream, k=k, v=v)
+    hip.check(hip.mi_hip_attn_fwd_reference_order(ctypes.byref(a)))
+    for j in (0, 1, 14, 15, 27, 28, 55, 56, 63, 64, 111, 112, 127, 128, 300, n_tok - 1):
+        one = torch.full((1, 1, d), float("nan"), device="cuda")
+        a = mh.attn_args(q[j:j + 1], one, 1, j, scale, stream, k=k, v=v)
+        hip.check(hip.mi_hip_attn_fwd_reference_order(ctypes.byref(a)))
+        torch.cuda.synchronize()
+        assert torch.equal(out[j].view(torch.int32), one[0].view(torch.int32)), j
