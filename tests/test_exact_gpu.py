@@ -134,11 +134,13 @@ def test_random_shapes_bit_for_bit(hip, stream, case):
     (1, 2, 128, 32767, 1),
     (1, 1, 64, 0, 300),      # more rows than workgroups and up to 300 keys: tiles
     (2, 7, 64, 63, 37),      # more rows than workgroups and few keys: staged, several a CU
-    (2, 7, 64, 55, 73),      # 128 keys, and more rows than run at once: tiles
-    (2, 7, 64, 56, 73),      # one key more: across a tile's edge
+    (2, 7, 64, 55, 73),      # 1022 rows of up to 128 keys: the last that run staged at once
+    (2, 7, 64, 54, 74),      # 1036 rows: tiles, rows past the last
+    (2, 7, 64, 55, 74),      # one key more: across a tile's edge
     (3, 5, 128, 3, 51),      # head_dim 128: 765 rows staged,
     (3, 5, 128, 3, 52),      # 780 in tiles, rows past the last
-    (3, 5, 128, 60, 20),     # head_dim 128, 100 rows per KV head
+    (3, 5, 128, 40, 60),     # across a tile's edge
+    (3, 5, 128, 60, 20),     # 300 staged, 100 rows per KV head
     (1, 8, 64, 4300, 40),    # more rows than workgroups, scores too long for tiles of 8 rows
     (3, 6, 64, 4090, 30),    # more than two rounds of them: tiles of 4
     (2, 9, 64, 4090, 70),    # more than one round of those: a wave per row

@@ -86,10 +86,11 @@ def test_q8_0_reproduces_reference_goldens(hip, stream, golden_manifest):
     (896, 896, 7),
     (896, 4864, 1),     # ffn_gate / ffn_up
     (4864, 896, 2),     # ffn_down
-    (896, 131, 13),     # rows not a multiple of 32, two column chunks
+    (896, 131, 13),     # rows and columns not multiples of a tile
     (3584, 512, 1),     # Qwen2.5-7B hidden size
     (896, 1152, 128),   # a 128-token prompt through the stacked Q/K/V rows
-    (96, 9, 2),         # odd block count: 102-byte rows end mid-dword (staged form)
+    (96, 9, 2),         # odd block count: 102-byte rows end mid-dword
+    (96, 9, 1),         # (one column: the staged form)
     (4832, 75, 1),      # 151 blocks per row, a 3-row last group
 ])
 def test_q8_0_model_shapes_equal_oracle(hip, stream, oracle, k, n, m):
@@ -104,12 +105,12 @@ def test_q8_0_model_shapes_equal_oracle(hip, stream, oracle, k, n, m):
     assert np.array_equal(bits(got), bits(want))
 
 
-@pytest.mark.parametrize("k,n,m", [(896, 100, 3), (4864, 61, 3)])
+@pytest.mark.parametrize("k,n,m", [(896, 100, 3), (4864, 61, 3), (896, 100, 1), (4864, 61, 1)])
 def test_q8_0_strided_operands(hip, stream, oracle, k, n, m):
     # padded weight rows, padded activation columns, a destination column
-    # stride wider than n: only the owned bytes are read or written (the
-    # second shape takes the LDS-staged form, whose last group ends at its
-    # last row's last block, not at the padded stride)
+    # stride wider than n: only the owned bytes are read or written (one
+    # column takes the LDS-staged form, whose last group ends at its last
+    # row's last block, not at the padded stride)
     import torch
     rng = np.random.default_rng(77)
     w = q8_weights(rng, n, k, w_nb1=k // 32 * 34 + 6)
