@@ -20,7 +20,7 @@
  * cosines and sines tabulated at load by the host's own cosf/sinf) and SiLU
  * (the host's expf, restated bit for bit) are bit-exact with the reference;
  * the attention is bit-exact in MI_HIP_QWEN2_ATTN_REFERENCE_ORDER mode and
- * within 1e-4 in the default fused mode.
+ * within 1e-4 in MI_HIP_QWEN2_ATTN_FUSED mode.
  *
  * Conventions as in mi_hip_attn.h: int status (MI_HIP_OK == 0), message in
  * mi_hip_last_error(); mi_hip_init must have been called. Host pointers are
@@ -97,8 +97,7 @@ int mi_hip_qwen2_generate(mi_hip_qwen2* model, const int32_t* prompt, int32_t n_
  *     (split-KV decode, MFMA prefill; within 1e-4 of the reference ops, so
  *     greedy ids follow the reference engine's until a near-tie argmax).
  *     The default when n_ctx > 32768.
- *   MI_HIP_QWEN2_ATTN_REFERENCE_ORDER (the default for n_ctx <= 32768): one
- *     wave per (token, head) running the
+ *   MI_HIP_QWEN2_ATTN_REFERENCE_ORDER (the default for n_ctx <= 32768): the
  *     reference's own operation order (src/ops_cpu.cpp:304-410: ordered dot
  *     products and sums, the C library's expf), bit-identical to the engine;
  *     cost linear in the context per row. With it every step of a forward call
